@@ -33,6 +33,7 @@ struct Sys {
   const double* kac0;
   const double* occ;
   double* rows;  // (NKB, 8)
+  double* rrows; // (kResSteps, NKB, 8), resident kernel
   int NK, NB, NKB, zb;
   int sw_zb, sw_tw;          // persistent sweep: column length along z, waves per team
   const int* kb_order;       // persistent sweep: atoms grouped by colour (no shared grid point within a colour)

@@ -8,6 +8,7 @@
 #include <algorithm>
 
 #include "batch_sweep.hpp"
+#include "resident.hpp"
 
 using namespace salmon::batch;
 
@@ -35,6 +36,17 @@ struct salmon_batch {
   int2* d_items = nullptr;        // (system, first orbital), costliest first (in bufs)
   int nitems = 0;
   int* d_next = nullptr;          // work counter of the sweep launch
+  // batches of systems whose orbitals fit in LDS (resident.hpp): one launch per
+  // workgroup shape (device memory in bufs)
+  struct ResClass {
+    int px = 0, waves = 0;
+    size_t lds = 0;
+    const int2* items = nullptr;  // (system, orbital)
+    int nitems = 0;
+  };
+  std::vector<ResClass> res;
+  const ResTab* d_restab = nullptr;
+  bool resident = false;
   unsigned sweep_grid = 0;
   size_t sweep_lds = 0;
   // one Taylor step at caller-given k points (batch_taylor): descriptors whose
@@ -77,6 +89,9 @@ static void batch_release(salmon_batch* b) {
   for (int ph = 0; ph < kPhases; ++ph) b->d_owner[ph] = nullptr;
   b->d_items = nullptr;
   b->nitems = 0;
+  b->res.clear();
+  b->d_restab = nullptr;
+  b->resident = false;
   b->sweep = false;
   b->ready = false;
 }
@@ -105,6 +120,159 @@ static std::array<int, 2> sweep_shape(const Grid& g) {
     }
   }
   return best;
+}
+
+// The resident kernel's plan: taken where it covers every system of the batch
+// (a grid of its shapes whose orbital, with the sphere points' tables, fits in
+// LDS, up to kResLpa projectors per atom, images within two cells) and the
+// orbitals are at most kResRounds per compute unit.  It runs one workgroup per
+// compute unit, so its time is about 10 (8^3) to 60 (16^3) us a step times the
+// rounds; the sweep's is nearly flat up to there (70 to 330 us for up to 256
+// orbitals) and then grows more slowly.  Beside systems that need the sweep the
+// sweep takes all: its work queue fills the chip across systems.  Builds the
+// tables, work lists and rows; b->resident stays false if the plan does not apply.
+constexpr int kResSteps = 32;  // steps per launch (rows kept per orbital)
+constexpr long kResRounds = 4;
+template <typename T>
+static int resident_plan(salmon_batch* b, std::vector<Sys<T>>& S) {
+  int dev = 0, ncu = 0;
+  BHIP(b, hipGetDevice(&dev));
+  BHIP(b, hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
+  long orbitals = 0;
+  for (const auto& y : S) {
+    orbitals += y.NKB;
+    const Grid& g = y.g;
+    if (!res_px(g) || res_lds<T>(g, y.kb.NPI, y.kb.NI) > kResMaxLds || y.kb.max_lpa > kResLpa || y.kb.NPI >= 0xffff ||
+        std::max({g.NLx, g.NLy, g.NLz}) > 200)
+      return SALMON_OK;
+  }
+  if (orbitals > kResRounds * ncu) return SALMON_OK;
+  // all tables and work lists in one device block: offsets first, pointers after its allocation
+  std::vector<unsigned char> blob;
+  auto put = [&](const void* src, size_t bytes) {
+    const size_t at = blob.size();
+    blob.resize((at + bytes + 15) / 16 * 16);
+    if (bytes) std::memcpy(blob.data() + at, src, bytes);
+    return at;
+  };
+  std::vector<std::array<size_t, 6>> at(S.size());
+  std::vector<int> nov(S.size());
+  std::vector<std::vector<int2>> items;
+  std::vector<salmon_batch::ResClass> res;
+  size_t rows = 0;
+  for (size_t i = 0; i < S.size(); ++i) {
+    const Grid& g = S[i].g;
+    const KBTables& kb = S[i].kb;
+    const auto& h = b->ctx[i]->kb_host;
+    std::vector<int> code(kb.NPI), prim(g.NL, kb.NPI), ovs(1, 0), ovj;
+    std::vector<double> uvp((size_t)kb.NPI * kResLpa, 0.0), sgp((size_t)kb.NI * kResLpa, 0.0);
+    for (int a = 0; a < kb.NI; ++a)
+      for (int l = h.lma[a]; l < h.lma[a + 1]; ++l) {
+        sgp[(size_t)a * kResLpa + l - h.lma[a]] = h.sign[l];
+        for (int jp = h.start[a]; jp < h.start[a + 1]; ++jp)
+          uvp[(size_t)jp * kResLpa + l - h.lma[a]] = h.uv[(size_t)l * kb.Nps + jp - h.start[a]];
+      }
+    const int N[3] = {g.NLx, g.NLy, g.NLz};
+    const double H[3] = {g.Hx, g.Hy, g.Hz}, L[3] = {g.aLx, g.aLy, g.aLz};
+    std::vector<int> more(kb.NPI, -1), last(g.NL, -1);  // sphere points of a grid point: prim, then chained in order
+    for (int jp = 0; jp < kb.NPI; ++jp) {
+      const int p = h.pidx[jp], l[3] = {p / (g.NLy * g.NLz), (p / g.NLz) % g.NLy, p % g.NLz};
+      if (last[p] < 0) prim[p] = jp;
+      else more[last[p]] = jp;
+      last[p] = jp;
+      code[jp] = 0;
+      for (int d = 0; d < 3; ++d) {
+        const int img = (int)std::lround((l[d] * H[d] - h.pos[3 * (size_t)jp + d]) / L[d]);  // pos = l H - img L
+        if (img < -2 || img > 2) return SALMON_OK;
+        code[jp] |= ((img + 2) * N[d] + l[d]) << (10 * d);
+      }
+    }
+    for (int p = 0; p < g.NL; ++p) {
+      if (prim[p] == kb.NPI || more[prim[p]] < 0) continue;
+      for (int jp = prim[p]; jp >= 0; jp = more[jp]) ovj.push_back(jp);
+      ovs.push_back((int)ovj.size());
+    }
+    nov[i] = (int)ovs.size() - 1;
+    at[i] = {put(prim.data(), sizeof(int) * prim.size()), put(code.data(), sizeof(int) * code.size()),
+             put(uvp.data(), sizeof(double) * uvp.size()), put(sgp.data(), sizeof(double) * sgp.size()),
+             put(ovs.data(), sizeof(int) * ovs.size()), put(ovj.data(), sizeof(int) * ovj.size())};
+    rows += (size_t)8 * kResSteps * S[i].NKB;
+    const int px = res_px(g), waves = res_waves(g, px);
+    size_t c = 0;
+    while (c < res.size() && (res[c].px != px || res[c].waves != waves)) ++c;
+    if (c == res.size()) {
+      res.emplace_back();
+      res[c].px = px;
+      res[c].waves = waves;
+      items.emplace_back();
+    }
+    res[c].lds = std::max(res[c].lds, res_lds<T>(g, kb.NPI, kb.NI));
+    for (int o = 0; o < S[i].NKB; ++o) items[c].push_back(int2{(int)i, o});
+  }
+  std::vector<size_t> at_items(res.size());
+  for (size_t c = 0; c < res.size(); ++c) at_items[c] = put(items[c].data(), sizeof(int2) * items[c].size());
+  std::vector<ResTab> tabs(S.size());
+  const size_t at_tabs = put(tabs.data(), sizeof(ResTab) * tabs.size());
+  unsigned char* d = nullptr;
+  double* d_rows = nullptr;
+  if (hipMalloc((void**)&d, blob.size()) != hipSuccess) return bfail(b, SALMON_ERR_NOMEM, "resident tables");
+  b->bufs.push_back(d);
+  if (hipMalloc((void**)&d_rows, sizeof(double) * rows) != hipSuccess)
+    return bfail(b, SALMON_ERR_NOMEM, "resident rows");
+  b->bufs.push_back(d_rows);
+  for (size_t i = 0; i < S.size(); ++i) {
+    tabs[i] = ResTab{(const int*)(d + at[i][0]), (const int*)(d + at[i][1]), (const double*)(d + at[i][2]),
+                     (const double*)(d + at[i][3]), (const int*)(d + at[i][4]), (const int*)(d + at[i][5]), nov[i], {}, {}};
+    for (int a = 0; a < 3; ++a)
+      for (int m = 0; m < 4; ++m) {
+        tabs[i].cc[a][m] = -0.5 * S[i].g.lap[a][m + 1];
+        tabs[i].dc[a][m] = S[i].g.nab[a][m + 1];
+      }
+    S[i].rrows = d_rows;
+    d_rows += (size_t)8 * kResSteps * S[i].NKB;
+  }
+  std::memcpy(blob.data() + at_tabs, tabs.data(), sizeof(ResTab) * tabs.size());
+  BHIP(b, hipMemcpy(d, blob.data(), blob.size(), hipMemcpyHostToDevice));
+  for (size_t c = 0; c < res.size(); ++c) {
+    res[c].nitems = (int)items[c].size();
+    res[c].items = (const int2*)(d + at_items[c]);
+  }
+  b->d_restab = (const ResTab*)(d + at_tabs);
+  b->res = res;
+  b->resident = true;
+  return SALMON_OK;
+}
+
+template <typename T, int PX>
+static int resident_launch_px(salmon_batch* b, const salmon_batch::ResClass& c, const Sys<T>* S, const ResArgs& a) {
+  // set once per kernel instantiation (a thread-safe static initialisation)
+  static const hipError_t attr = hipFuncSetAttribute((const void*)k_b_resident<T, PX>,
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)kResMaxLds);
+  BHIP(b, attr);
+  hipLaunchKernelGGL((k_b_resident<T, PX>), dim3(c.nitems), dim3(c.waves * kWave), c.lds, b->stream, S,
+                     b->d_restab, c.items, a);
+  return SALMON_OK;
+}
+
+// Steps n0 .. n0 + a.nsteps - 1 (at most kResSteps) of a resident batch, and with
+// a.obs their sums into res.
+template <typename T>
+static int resident_launch(salmon_batch* b, const Sys<T>* S, const ResArgs& a, double* res) {
+  int r = SALMON_OK;
+  for (const auto& c : b->res) {
+    switch (c.px) {
+      case 1: r = resident_launch_px<T, 1>(b, c, S, a); break;
+      case 2: r = resident_launch_px<T, 2>(b, c, S, a); break;
+      case 3: r = resident_launch_px<T, 3>(b, c, S, a); break;
+      case 4: r = resident_launch_px<T, 4>(b, c, S, a); break;
+      default: r = resident_launch_px<T, 6>(b, c, S, a); break;
+    }
+    if (r) return r;
+  }
+  if (a.obs)
+    hipLaunchKernelGGL(k_b_resident_sum<T>, dim3((unsigned)b->ctx.size(), a.nsteps), dim3(256), 0, b->stream, S, a.n0, res);
+  BHIP(b, hipGetLastError());
+  return SALMON_OK;
 }
 
 // The persistent sweep's work list, LDS size and grid; b->sweep stays false
@@ -142,9 +310,7 @@ static int sweep_plan(salmon_batch* b, std::vector<Sys<T>>& S) {
   for (size_t i = 0; i < S.size(); ++i) {
     const KBTables& kb = S[i].kb;
     if (kb.NI <= 0 || kb.Nlma <= 0) continue;
-    std::vector<int> ast(kb.NI + 1), pidx(std::max(1, kb.NPI));
-    BHIP(b, hipMemcpy(ast.data(), kb.atom_start, sizeof(int) * (kb.NI + 1), hipMemcpyDeviceToHost));
-    if (kb.NPI > 0) BHIP(b, hipMemcpy(pidx.data(), kb.pidx, sizeof(int) * kb.NPI, hipMemcpyDeviceToHost));
+    const std::vector<int>&ast = b->ctx[i]->kb_host.start, &pidx = b->ctx[i]->kb_host.pidx;
     std::vector<std::vector<char>> used;
     std::vector<int> colour(kb.NI);
     for (int a = 0; a < kb.NI; ++a) {
@@ -217,10 +383,11 @@ static int batch_build(salmon_batch* b) {
   const int n = (int)b->ctx.size();
   std::vector<Sys<T>> S(n);
   b->max_ph = 0;
-  long acc[kPhases] = {0, 0, 0, 0, 0};
+  bool sweeps = b->kernel_req != SALMON_BATCH_PHASES;
   for (int i = 0; i < n; ++i) {
     salmon_ctx* c = b->ctx[i];
     Sys<T>& y = S[i];
+    sweeps = sweeps && sweep_shape<T>(c->g)[0] > 0;
     y.g = c->g;
     y.kb = c->kb;
     y.zu = (cplx<T>*)c->d_zu;
@@ -233,6 +400,14 @@ static int batch_build(salmon_batch* b) {
     y.NKB = c->NKB;
     y.zb = b->zb[i];
     y.sw_zb = y.sw_tw = 0;
+    y.rrows = nullptr;
+  }
+  int r;
+  if (sweeps && (r = resident_plan<T>(b, S))) return r;
+  long acc[kPhases] = {0, 0, 0, 0, 0};
+  for (int i = 0; i < n && !b->resident; ++i) {
+    salmon_ctx* c = b->ctx[i];
+    Sys<T>& y = S[i];
     const size_t nv = (size_t)c->NKB * c->g.NL;
     for (int t = 0; t < 4; ++t) {
       if (hipMalloc((void**)&y.h[t], nv * sizeof(cplx<T>)) != hipSuccess)
@@ -266,7 +441,7 @@ static int batch_build(salmon_batch* b) {
   // stencil blocks class by class, so that one launch per z blocking covers
   // every system of the class
   const int zbs[4] = {1, 2, 4, 8};
-  for (int k = 0; k < 4; ++k) {
+  for (int k = 0; k < 4 && !b->resident; ++k) {
     b->zcls[k][0] = acc[1];
     for (int i = 0; i < n; ++i) {
       if (S[i].zb != zbs[k]) continue;
@@ -275,7 +450,7 @@ static int batch_build(salmon_batch* b) {
     }
     b->zcls[k][1] = acc[1] - b->zcls[k][0];
   }
-  for (int ph = 0; ph < kPhases; ++ph) {
+  for (int ph = 0; ph < kPhases && !b->resident; ++ph) {
     b->first[ph].assign(1, acc[ph]);
     std::vector<unsigned short> own((size_t)acc[ph]);
     for (int i = 0; i < n; ++i) {
@@ -290,8 +465,8 @@ static int batch_build(salmon_batch* b) {
     b->bufs.push_back(b->d_owner[ph]);
     BHIP(b, hipMemcpy(b->d_owner[ph], own.data(), sizeof(unsigned short) * own.size(), hipMemcpyHostToDevice));
   }
-  int r = sweep_plan<T>(b, S);
-  if (r) return r;
+  b->sweep = b->resident;
+  if (!b->resident && (r = sweep_plan<T>(b, S))) return r;
   if (hipMalloc(&b->d_sys, sizeof(Sys<T>) * n) != hipSuccess) return bfail(b, SALMON_ERR_NOMEM, "batch descriptors");
   b->bufs.push_back(b->d_sys);
   BHIP(b, hipMemcpy(b->d_sys, S.data(), sizeof(Sys<T>) * n, hipMemcpyHostToDevice));
@@ -398,6 +573,7 @@ static int batch_taylor(salmon_batch* b, const double* const* kbase, double dt) 
   int r;
   if ((r = batch_k_descriptors<T>(b, kbase))) return r;
   const Sys<T>* S = (const Sys<T>*)b->d_sys_k;
+  if (b->resident) return resident_launch<T>(b, S, ResArgs{nullptr, 0L, 0, 1, dt, 1, 0}, nullptr);
   const Step st{b->d_zero_ac, b->d_zero_step, dt,
                 {b->d_owner[0], b->d_owner[1], b->d_owner[2], b->d_owner[3], b->d_owner[4]}, 0L};
   if (b->max_ph > 0)
@@ -425,14 +601,18 @@ static int batch_observe(salmon_batch* b, const double* const* kbase, double* ou
     b->exec = nullptr;
   }
   const Sys<T>* S = (const Sys<T>*)b->d_sys_k;
-  const Step st{b->d_zero_ac, b->d_zero_step, 0.0,
-                {b->d_owner[0], b->d_owner[1], b->d_owner[2], b->d_owner[3], b->d_owner[4]}, 0L, 1};
-  if (b->max_ph > 0)
-    hipLaunchKernelGGL(k_b_phase<T>, dim3((unsigned)((b->max_ph + 255) / 256), n), dim3(256), 0, b->stream, S, st, 2);
-  hipLaunchKernelGGL(k_b_qreset, dim3(1), dim3(64), 0, b->stream, b->d_next);
-  batch_sweep_launch<T>(b, S, st);
-  hipLaunchKernelGGL(k_b_sum<T>, dim3(n), dim3(256), 0, b->stream, S, n, b->d_zero_step, b->d_res, 0);
-  BHIP(b, hipGetLastError());
+  if (b->resident) {
+    if ((r = resident_launch<T>(b, S, ResArgs{nullptr, 0L, 0, 1, 0.0, 0, 1}, b->d_res))) return r;
+  } else {
+    const Step st{b->d_zero_ac, b->d_zero_step, 0.0,
+                  {b->d_owner[0], b->d_owner[1], b->d_owner[2], b->d_owner[3], b->d_owner[4]}, 0L, 1};
+    if (b->max_ph > 0)
+      hipLaunchKernelGGL(k_b_phase<T>, dim3((unsigned)((b->max_ph + 255) / 256), n), dim3(256), 0, b->stream, S, st, 2);
+    hipLaunchKernelGGL(k_b_qreset, dim3(1), dim3(64), 0, b->stream, b->d_next);
+    batch_sweep_launch<T>(b, S, st);
+    hipLaunchKernelGGL(k_b_sum<T>, dim3(n), dim3(256), 0, b->stream, S, n, b->d_zero_step, b->d_res, 0);
+    BHIP(b, hipGetLastError());
+  }
   BHIP(b, hipMemcpyAsync(out, b->d_res, sizeof(double) * 8 * (size_t)n, hipMemcpyDeviceToHost, b->stream));
   BHIP(b, hipStreamSynchronize(b->stream));
   return SALMON_OK;
@@ -587,12 +767,19 @@ static int batch_run(salmon_batch* b, const double* ac, int nsteps, double dt, d
     b->exec = nullptr;
   }
   BHIP(b, hipMemcpyAsync(b->d_ac, ac, sizeof(double) * need_ac, hipMemcpyHostToDevice, b->stream));
-  BHIP(b, hipMemsetAsync(b->d_step, 0, sizeof(int), b->stream));
+  // a resident batch: kResSteps steps per launch, straight from the A(t) tables
+  if (b->resident)
+    for (int s = 0; s < nsteps; s += kResSteps) {
+      const ResArgs a{b->d_ac, stride, s, std::min(kResSteps, nsteps - s), dt, 1, 1};
+      if ((r = resident_launch<T>(b, (const Sys<T>*)b->d_sys, a, b->d_res))) return r;
+    }
+  const bool graph_steps = !b->resident;
+  if (graph_steps) BHIP(b, hipMemsetAsync(b->d_step, 0, sizeof(int), b->stream));
   if (b->exec && (b->graph_dt != dt || b->graph_stride != stride)) {
     (void)hipGraphExecDestroy(b->exec);
     b->exec = nullptr;
   }
-  if (!b->exec) {
+  if (graph_steps && !b->exec) {
     hipGraph_t graph = nullptr;
     BHIP(b, hipStreamBeginCapture(b->stream, hipStreamCaptureModeRelaxed));
     r = batch_enqueue_step<T>(b, dt, stride);
@@ -608,8 +795,9 @@ static int batch_run(salmon_batch* b, const double* ac, int nsteps, double dt, d
     b->graph_dt = dt;
     b->graph_stride = stride;
   }
-  for (int s = 0; s < nsteps; ++s) BHIP(b, hipGraphLaunch(b->exec, b->stream));
-  if (b->sweep && (r = batch_close_sweep<T>(b, dt, stride))) return r;
+  if (graph_steps)
+    for (int s = 0; s < nsteps; ++s) BHIP(b, hipGraphLaunch(b->exec, b->stream));
+  if (graph_steps && b->sweep && (r = batch_close_sweep<T>(b, dt, stride))) return r;
   std::vector<double> res(8 * (size_t)n * nsteps);
   BHIP(b, hipMemcpyAsync(res.data(), b->d_res, sizeof(double) * res.size(), hipMemcpyDeviceToHost, b->stream));
   BHIP(b, hipStreamSynchronize(b->stream));

@@ -51,6 +51,10 @@ struct salmon_ctx {
   bool have_kb = false;
   KBTables kb{};
   std::vector<void*> kb_bufs;
+  struct {  // the same tables on the host, for the plans built from them
+    std::vector<int> start, pidx, lma;
+    std::vector<double> pos, uv, sign;
+  } kb_host;
   // k points / orbitals
   int NK = 0, NB = 0, NKB = 0;
   double* d_kac0 = nullptr;   // (3*NK) as kAc0(NK,3)
@@ -1064,6 +1068,7 @@ int salmon_gpu_set_projectors(salmon_ctx* c, int NI, int Nps, const int* Mps, co
       (r = up(ejp.data(), sizeof(int) * ejp.size(), (void**)&kb.e_jp)))
     return r;
   c->kb = kb;
+  c->kb_host = {start, pidx, atom_lma, pos, std::vector<double>(uV, uV + (size_t)Nps * Nlma), sign};
   c->have_kb = true;
   dfree(&c->d_uvpsi);
   for (int i = 0; i < 4; ++i) dfree(&c->d_work[i]);
