@@ -5,6 +5,7 @@
 // frozen potential.  Included by salmon_gpu.hip after its helpers.
 #pragma once
 #include "cg.hpp"
+#include "gsblock.hpp"
 
 using namespace salmon::cg;
 
@@ -35,6 +36,7 @@ struct GsState {
   double* tw = nullptr;    // DFT twiddles (3*kDftMax complex)
   double* symb = nullptr;  // kinetic symbol per axis (3*kDftMax)
   int pstride = 0;
+  GsBlock gsb{};  // panel Gram-Schmidt
   // subspace matrices
   double* dpart = nullptr;
   size_t dpart_n = 0;
@@ -148,6 +150,24 @@ static int gs_ensure(salmon_ctx* c) {
   if ((r = gs_alloc(c, s, &s->minvr, (size_t)s->NK * s->NB * s->NB))) return r;
   if ((r = gs_alloc(c, s, &s->tw, (size_t)2 * 3 * kDftMax))) return r;
   if ((r = gs_alloc(c, s, &s->symb, (size_t)3 * kDftMax))) return r;
+  GsBlock& q = s->gsb;
+  q.NK = s->NK;
+  q.NB = s->NB;
+  q.NL = s->NL;
+  q.Hxyz = c->g.Hxyz;
+  q.ntile = (s->NB + kPanel - 1) / kPanel;
+  // about 1024 blocks, chunks of at least 1024 points: each 64 bands x 32^3 sweep took 44.4 ms
+  // with 1024, 44.5 with 512 and 44.8 with 2048; ten steps of 276 x 20x20x28, reorthonormalised
+  // every fifth, 3.30, 3.42 and 3.33
+  q.nchunk = std::max(1, std::min(1024 / (s->NK * q.ntile), (s->NL + 1023) / 1024));
+  q.chunk = ((s->NL + q.nchunk - 1) / q.nchunk + 63) / 64 * 64;
+  q.nchunk = (s->NL + q.chunk - 1) / q.chunk;
+  if ((r = gs_alloc(c, s, &q.part, (size_t)s->NK * q.ntile * q.nchunk * 256))) return r;
+  if ((r = gs_alloc(c, s, &q.C, (size_t)s->NK * s->NB * kPanel))) return r;
+  if ((r = gs_alloc(c, s, &q.W, (size_t)s->NK * s->NB * kPanel))) return r;
+  if ((r = gs_alloc(c, s, &q.cnt, (size_t)s->NK * (q.ntile + 1)))) return r;
+  if ((r = gs_alloc(c, s, &q.flag, s->NK))) return r;
+  HIPCHK(c, hipMemsetAsync(q.cnt, 0, sizeof(unsigned) * s->NK * (q.ntile + 1), c->stream));
   HIPCHK(c, hipMemsetAsync(s->cnt, 0, sizeof(unsigned) * s->NK, c->stream));
   HIPCHK(c, hipMemsetAsync(s->sc, 0, sizeof(double) * s->NK * kNS, c->stream));
   HIPCHK(c, hipMemsetAsync(s->done, 0, sizeof(int) * s->NK, c->stream));
@@ -325,6 +345,31 @@ static int gram_schmidt_multi(salmon_ctx* c, cplx<double>* zu) {
     hipLaunchKernelGGL(k_gs_scale, gv, blk, 0, c->stream, S, zu, ib);
     LAUNCHCHK(c);
   }
+  return SALMON_OK;
+}
+
+// Gram_Schmidt_ompk in panels (gsblock.hpp); *done = 0 if a panel could not be
+// orthogonalised so (waits for the stream).
+static int gram_schmidt_panels(salmon_ctx* c, cplx<double>* zu, int* done) {
+  int r;
+  if ((r = gs_ensure(c))) return r;
+  GsState* s = (GsState*)c->gs;
+  GsBlock b = s->gsb;
+  b.zu = zu;
+  HIPCHK(c, hipMemsetAsync(b.flag, 0, sizeof(int) * b.NK, c->stream));
+  for (int j0 = 0; j0 < b.NB; j0 += kPanel) {
+    const int np = std::min(kPanel, b.NB - j0);
+    for (int round = 0; round < 2; ++round) {
+      hipLaunchKernelGGL(k_gsb_overlap, dim3(b.nchunk, (j0 + np + kPanel - 1) / kPanel, b.NK), dim3(256), 0, c->stream, b,
+                         j0, np);
+      hipLaunchKernelGGL(k_gsb_apply, dim3((b.NL + 63) / 64, b.NK), dim3(256), 0, c->stream, b, j0, np);
+      LAUNCHCHK(c);
+    }
+  }
+  std::vector<int> flag(b.NK);
+  HIPCHK(c, hipMemcpyAsync(flag.data(), b.flag, sizeof(int) * b.NK, hipMemcpyDeviceToHost, c->stream));
+  HIPCHK(c, hipStreamSynchronize(c->stream));
+  *done = std::all_of(flag.begin(), flag.end(), [](int f) { return f == 0; });
   return SALMON_OK;
 }
 

@@ -476,6 +476,9 @@ namespace {
 int gram_schmidt_multi_fwd(salmon_ctx* c, cplx<double>* zu) {
   int r = ensure_work(c);
   if (r || (r = gs_ensure(c))) return r;
+  int done = 0;
+  if ((r = gram_schmidt_panels(c, zu, &done)) || done) return r;
+  // nearly dependent (or not finite) bands: band by band
   GsState* s = (GsState*)c->gs;
   const long key[4] = {(long)(uintptr_t)zu, c->NB, c->NK, 0};
   return graph_run(c, s->g_gs, key, [&]() { return gram_schmidt_multi(c, zu); });
