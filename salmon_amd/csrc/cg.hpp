@@ -12,28 +12,19 @@
 // A k whose band met the exit test (|ev - <x|H|x>| < 1e-15, CG.f90:114)
 // skips the remaining iteration kernels.
 #pragma once
-#include "common.hpp"
+#include "streamed.hpp"
 
 namespace salmon {
 namespace cg {
 
-#ifndef SALMON_CG_PPT
-#define SALMON_CG_PPT 4
-#endif
-constexpr int kPPT = SALMON_CG_PPT;  // points per thread per chunk
-constexpr int kChunk = 256 * kPPT;   // points per block
-// the lower-band subtractions (k_cg_sub, k_gs_sub) read ib bands per point and
-// run on finer chunks: more workgroups keep more of those loads in flight
-#ifndef SALMON_CG_SUB_PPT
-#define SALMON_CG_SUB_PPT 1
-#endif
-constexpr int kSubPPT = SALMON_CG_SUB_PPT;
-constexpr int kSubChunk = 256 * kSubPPT;
+constexpr int kPPT = 2;              // points per thread of a projection block
+constexpr int kChunk = 256 * kPPT;   // points per projection block
 constexpr int kJG = 8;               // lower bands per projection block
+constexpr int kSubPts = 64;          // points per subtraction block, one per lane; its waves share the bands
 
 // per-k scalars (double slots)
 enum : int {
-  XHX = 0, XTX, GKGK, UK, SN, EVX, CXR, CXI, CP, ZSR, ZSI, EFIN, kNS = 16
+  XHX = 0, XTX, GKGK, UK, SN, EVX, CXR, CXI, CP, ZSR, ZSI, EFIN, XN, kNS = 16
 };
 
 struct State {
@@ -48,16 +39,19 @@ struct State {
   cplx<double>* minv;  // (NK*NB*NB) rows of (I + L)^-1, L(j,i) = G(j,i) for i < j
   double* minvr;       // (NK*NB*NB) rows of (I + Re L)^-1
   const double* occ; // (NK*NB)
-  int NK, NB, NL, nchunk;
-  int nsub;          // chunks of the subtraction kernels (kSubChunk points)
-  int pstride;       // doubles of part per k: nchunk*ceil(NB/kJG)*kPartQ
+  int NK, NB, NL;
+  int nchunk;        // blocks of a projection (kChunk points)
+  int nsub;          // blocks of a subtraction (kSubPts points)
+  int nvec;          // blocks of the other kernels (256 points)
+  int pstride;       // doubles of part per k
   double Hxyz;
 };
 constexpr int kPartQ = 2 * kJG;
 
-// Sums NQ per-block values over the blocks of row k = blockIdx.y in block
+// Sums NQ per-block values over the nblk blocks of row k = blockIdx.y in a fixed
 // order.  Returns true in the block that arrives last; there, tot[] holds the
-// totals in thread 0.  nblk = number of blocks of the row.
+// totals in thread 0.  Its threads load the partials side by side: one thread
+// reading them in block order took 1 to 3 us per launch on 32 to 128 blocks.
 template <int NQ>
 __device__ bool last_block_sum(double (&v)[NQ], const State& S, int nblk, int bid, double (&tot)[NQ]) {
   __shared__ double smem[4 * NQ];
@@ -68,23 +62,26 @@ __device__ bool last_block_sum(double (&v)[NQ], const State& S, int nblk, int bi
   if (threadIdx.x == 0) {
 #pragma unroll
     for (int q = 0; q < NQ; ++q) __hip_atomic_store(&part[bid * NQ + q], v[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const unsigned t = __hip_atomic_fetch_add(&S.cnt[k], 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
+    agent_stores_done();
+    const unsigned t = agent_arrive(&S.cnt[k]);
     is_last = (t == (unsigned)(nblk - 1));
+    if (is_last) __hip_atomic_store(&S.cnt[k], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
   __syncthreads();
   if (!is_last) return false;
-  if (threadIdx.x == 0) {
 #pragma unroll
-    for (int q = 0; q < NQ; ++q) tot[q] = 0.0;
-#pragma unroll 8
-    for (int b = 0; b < nblk; ++b) {
+  for (int q = 0; q < NQ; ++q) tot[q] = 0.0;
+  for (int b = threadIdx.x; b < nblk; b += 256) {
 #pragma unroll
-      for (int q = 0; q < NQ; ++q) tot[q] += __hip_atomic_load(&part[b * NQ + q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    __hip_atomic_store(&S.cnt[k], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    for (int q = 0; q < NQ; ++q) tot[q] += __hip_atomic_load(&part[b * NQ + q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
+  block_sum256<NQ>(tot, smem);
   return true;
 }
+
+// Keeps the loads of v before this point.  The kernels look at the exit flag
+// after their loads, so that it does not add a memory round trip to each launch.
+__device__ __forceinline__ void loaded(const cplx<double>& v) { asm volatile("" ::"v"(v.re), "v"(v.im)); }
 
 __device__ __forceinline__ cplx<double> cmulc(cplx<double> a, cplx<double> b) {  // a*b
   return {a.re * b.re - a.im * b.im, a.re * b.im + a.im * b.re};
@@ -130,7 +127,7 @@ constexpr int kCgMaxNB = 1024;
 __global__ void __launch_bounds__(256) k_cg_proj(State S, const cplx<double>* __restrict__ zu, int ib, Src src,
                                                  int mode, int check_done) {
   const int k = blockIdx.z;
-  if (check_done && S.done[k]) return;
+  const int skip = check_done ? S.done[k] : 0;
   const int c = blockIdx.x, g0 = blockIdx.y * kJG;
   const int nj = min(kJG, ib - g0);
   const double xhx = S.sc[k * kNS + XHX];
@@ -171,105 +168,150 @@ __global__ void __launch_bounds__(256) k_cg_proj(State S, const cplx<double>* __
       acc[2 * j + 1] += br * e[i].im - bi * e[i].re;
     }
   }
-  __shared__ double smem[4 * 2 * kJG];
-  block_sum256<2 * kJG>(acc, smem);
-  // partials: [group][chunk][2*kJG]; the last block of row k sums over chunks
+  loaded(cplx<double>{acc[0], acc[2 * kJG - 1]});
+  if (skip) return;
+  // partials: [group][chunk][2*kJG]
+  __shared__ double smem[4 * kPartQ];
   __shared__ int is_last;
-  double* part = S.part + (size_t)k * S.pstride;
-  const int ngroup = gridDim.y, nblk = S.nchunk * ngroup;
-  const int bid = blockIdx.y * S.nchunk + c;
-  if (threadIdx.x == 0) {
+  const int t = threadIdx.x, lane = t & (kWave - 1), wv = t / kWave;
+  wave_sums(acc);
 #pragma unroll
-    for (int q = 0; q < 2 * kJG; ++q)
-      __hip_atomic_store(&part[(size_t)bid * kPartQ + q], acc[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const unsigned t = __hip_atomic_fetch_add(&S.cnt[k], 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
-    is_last = (t == (unsigned)(nblk - 1));
+  for (int q = 0; q < kPartQ; ++q)
+    if (lane == wave_sums_lane(q)) smem[wv * kPartQ + q] = acc[0];
+  double* part = S.part + (size_t)k * S.pstride;
+  const int nblk = S.nchunk * gridDim.y;
+  const int bid = blockIdx.y * S.nchunk + c;
+  __syncthreads();
+  if (wv == 0) {  // one wave stores them and arrives: its stores are ordered before its arrival
+    if (lane < kPartQ) {
+      const double v = (smem[lane] + smem[kPartQ + lane]) + (smem[2 * kPartQ + lane] + smem[3 * kPartQ + lane]);
+      __hip_atomic_store(&part[(size_t)bid * kPartQ + lane], v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    agent_stores_done();
+    if (lane == 0) {
+      const unsigned n = agent_arrive(&S.cnt[k]);
+      is_last = (n == (unsigned)(nblk - 1));
+      if (is_last) __hip_atomic_store(&S.cnt[k], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
   }
   __syncthreads();
   if (!is_last) return;
+  // The last block of row k: four threads per band (quad qd, part qi), each
+  // taking every fourth term of a sum with kTailBatch loads in flight (clamped
+  // indices, terms past the end zero), then the quad's sum in a fixed order.
+  // One thread per band left this to 64 lanes and up to 64 dependent loads.
   __shared__ cplx<double> zsh[kCgMaxNB];
-  // one thread per lower band sums its chunks in chunk order; the partials of
-  // kTailBatch chunks are loaded (clamped chunk index) before any is added,
-  // so one cache round trip serves the batch
-  constexpr int kTailBatch = 32;
-  for (int j = threadIdx.x; j < ib; j += 256) {
-    const int grp = j / kJG, jj = j % kJG;
+  constexpr int kTailBatch = 16;
+  const int qd = t >> 2, qi = t & 3;
+  auto quad = [](double v) {
+    v += dpp_mov<dpp::kQuad1032, 0xf>(v);
+    return v + dpp_mov<dpp::kQuad2301, 0xf>(v);
+  };
+  for (int j0 = 0; j0 < ib; j0 += 64) {
+    const int j = j0 + qd, jc = min(j, ib - 1), grp = jc / kJG, jj = jc % kJG;
     double sr = 0.0, si = 0.0;
-    for (int c0 = 0; c0 < S.nchunk; c0 += kTailBatch) {
+    for (int c0 = qi; c0 < S.nchunk; c0 += 4 * kTailBatch) {
       double vr[kTailBatch], vi[kTailBatch];
 #pragma unroll
       for (int u = 0; u < kTailBatch; ++u) {
-        const size_t b = (size_t)(grp * S.nchunk + min(c0 + u, S.nchunk - 1)) * kPartQ;
+        const size_t b = (size_t)(grp * S.nchunk + min(c0 + 4 * u, S.nchunk - 1)) * kPartQ;
         vr[u] = __hip_atomic_load(&part[b + 2 * jj], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         vi[u] = __hip_atomic_load(&part[b + 2 * jj + 1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       }
 #pragma unroll
       for (int u = 0; u < kTailBatch; ++u) {
-        const bool ok = c0 + u < S.nchunk;
+        const bool ok = c0 + 4 * u < S.nchunk;
         sr = ok ? sr + vr[u] : sr;
         si = ok ? si + vi[u] : si;
       }
     }
-    zsh[j] = cplx<double>{sr * S.Hxyz, si * S.Hxyz};
+    sr = quad(sr);
+    si = quad(si);
+    if (qi == 0 && j < ib) zsh[j] = cplx<double>{sr * S.Hxyz, si * S.Hxyz};
   }
-  if (threadIdx.x == 0) __hip_atomic_store(&S.cnt[k], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   __syncthreads();
   cplx<double>* gram = S.gram + (size_t)k * S.NB * S.NB;
   cplx<double>* M = S.minv + (size_t)k * S.NB * S.NB;
   double* MR = S.minvr + (size_t)k * S.NB * S.NB;
+  if (mode == PROJ_PLAIN) {  // coefficients against the unmodified vector
+    for (int j = t; j < ib; j += 256) S.zs[(size_t)k * S.NB + j] = zsh[j];
+    return;
+  }
   if (mode == PROJ_GRAM) {
     // raw_j = Hxyz <B_j|B_ib>, so G(ib, j) = conj(raw_j)
-    for (int j = threadIdx.x; j < ib; j += 256) gram[(size_t)ib * S.NB + j] = cplx<double>{zsh[j].re, -zsh[j].im};
+    for (int j = t; j < ib; j += 256) gram[(size_t)ib * S.NB + j] = cplx<double>{zsh[j].re, -zsh[j].im};
     // the unit diagonal of M is implicit (band 0 has no projection launch)
-    for (int l = threadIdx.x; l < ib; l += 256) {
-      double sr = zsh[l].re, si = -zsh[l].im, rr = zsh[l].re;  // q = l: G(ib, l) M(l, l)
-      for (int q = l + 1; q < ib; ++q) {
-        const double gr = zsh[q].re, gi = -zsh[q].im;
-        const cplx<double> m = M[(size_t)q * S.NB + l];
-        sr += gr * m.re - gi * m.im;
-        si += gr * m.im + gi * m.re;
-        rr += gr * MR[(size_t)q * S.NB + l];
+    for (int j0 = 0; j0 < ib; j0 += 64) {
+      const int l = j0 + qd, lc = min(l, ib - 1);
+      double sr = 0.0, si = 0.0, rr = 0.0;
+      if (qi == 0) {  // q = l: G(ib, l) M(l, l)
+        sr = rr = zsh[lc].re;
+        si = -zsh[lc].im;
       }
-      M[(size_t)ib * S.NB + l] = cplx<double>{-sr, -si};
-      MR[(size_t)ib * S.NB + l] = -rr;
-    }
-    return;
-  }
-  if (mode == PROJ_PLAIN) {  // coefficients against the unmodified vector
-    for (int j = threadIdx.x; j < ib; j += 256) S.zs[(size_t)k * S.NB + j] = zsh[j];
-    return;
-  }
-  // c = M b, one thread per row in column order; the row's entries of
-  // kTailBatch columns are loaded (clamped column index) before any is used
-  for (int j = threadIdx.x; j < ib; j += 256) {
-    double cr = zsh[j].re, ci = mode == PROJ_START ? 0.0 : zsh[j].im;
-    if (mode == PROJ_START) {
-      for (int l0 = 0; l0 < j; l0 += kTailBatch) {
+      for (int q0 = j0 + qi; q0 < ib; q0 += 4 * kTailBatch) {
+        cplx<double> mm[kTailBatch];
         double mr[kTailBatch];
 #pragma unroll
-        for (int u = 0; u < kTailBatch; ++u) mr[u] = MR[(size_t)j * S.NB + min(l0 + u, j - 1)];
+        for (int u = 0; u < kTailBatch; ++u) {
+          const size_t o = (size_t)max(min(q0 + 4 * u, ib - 1), lc) * S.NB + lc;  // (row q > column l, or not used)
+          mm[u] = M[o];
+          mr[u] = MR[o];
+        }
 #pragma unroll
         for (int u = 0; u < kTailBatch; ++u) {
-          const int l = l0 + u;
-          cr = l < j ? cr + mr[u] * zsh[min(l, j - 1)].re : cr;
+          const int q = q0 + 4 * u;
+          const bool ok = q > l && q < ib;
+          const cplx<double> z = zsh[min(q, ib - 1)];
+          sr = ok ? sr + (z.re * mm[u].re + z.im * mm[u].im) : sr;
+          si = ok ? si + (z.re * mm[u].im - z.im * mm[u].re) : si;
+          rr = ok ? rr + z.re * mr[u] : rr;
         }
       }
-    } else {
-      for (int l0 = 0; l0 < j; l0 += kTailBatch) {
-        cplx<double> mm[kTailBatch];
+      sr = quad(sr);
+      si = quad(si);
+      rr = quad(rr);
+      if (qi == 0 && l < ib) {
+        M[(size_t)ib * S.NB + l] = cplx<double>{-sr, -si};
+        MR[(size_t)ib * S.NB + l] = -rr;
+      }
+    }
+    return;
+  }
+  // c = M b
+  for (int j0 = 0; j0 < ib; j0 += 64) {
+    const int j = j0 + qd, jc = min(j, ib - 1);
+    double cr = 0.0, ci = 0.0;
+    if (qi == 0) {
+      cr = zsh[jc].re;
+      ci = mode == PROJ_START ? 0.0 : zsh[jc].im;
+    }
+    const int l1 = min(ib, j0 + 64);  // columns below the rows of this pass
+    for (int l0 = qi; l0 < l1; l0 += 4 * kTailBatch) {
+      if (mode == PROJ_START) {
+        double mr[kTailBatch];
 #pragma unroll
-        for (int u = 0; u < kTailBatch; ++u) mm[u] = M[(size_t)j * S.NB + min(l0 + u, j - 1)];
+        for (int u = 0; u < kTailBatch; ++u) mr[u] = MR[(size_t)jc * S.NB + min(l0 + 4 * u, jc)];
 #pragma unroll
         for (int u = 0; u < kTailBatch; ++u) {
-          const int l = l0 + u;
-          const cplx<double> m = mm[u], z = zsh[min(l, j - 1)];
-          const double tr = cr + (m.re * z.re - m.im * z.im), ti = ci + (m.re * z.im + m.im * z.re);
-          cr = l < j ? tr : cr;
-          ci = l < j ? ti : ci;
+          const int l = l0 + 4 * u;
+          cr = l < jc ? cr + mr[u] * zsh[min(l, jc)].re : cr;
+        }
+      } else {
+        cplx<double> mm[kTailBatch];
+#pragma unroll
+        for (int u = 0; u < kTailBatch; ++u) mm[u] = M[(size_t)jc * S.NB + min(l0 + 4 * u, jc)];
+#pragma unroll
+        for (int u = 0; u < kTailBatch; ++u) {
+          const int l = l0 + 4 * u;
+          const cplx<double> m = mm[u], z = zsh[min(l, jc)];
+          cr = l < jc ? cr + (m.re * z.re - m.im * z.im) : cr;
+          ci = l < jc ? ci + (m.re * z.im + m.im * z.re) : ci;
         }
       }
     }
-    S.zs[(size_t)k * S.NB + j] = cplx<double>{cr, ci};
+    cr = quad(cr);
+    ci = quad(ci);
+    if (qi == 0 && j < ib) S.zs[(size_t)k * S.NB + j] = cplx<double>{cr, ci};
   }
 }
 
@@ -285,297 +327,345 @@ enum : int {
 };
 
 // out = src - sum_{j<ib} zs(j) B_j  (CG.f90:69-71, 86-89), then the role's
-// reduction.  For SUB_GRAD / SUB_PCDIR the finisher forms the conjugation
-// ratio uk = s/gkgk (CG.f90:92-98; iteration 1 takes p = direction).
-// Grid (nsub, NK).
+// reduction.  For a search direction d (the roles but SUB_START and SUB_NONE) the
+// finisher forms the conjugation ratio uk = s/gkgk (CG.f90:92-98; iteration 1
+// takes p = d) and, from <x|d> and <x|p_old>, the overlap zs = <x|d + uk p_old>
+// that the direction is stripped of (CG.f90:103), so p needs no pass of its own.
+// A block's lanes are its points and its four waves take every fourth band: the
+// loop's loads are the launch's time (64 bands of 32^3: 8 loads in flight per
+// lane, two rounds of them instead of eight).  Grid (nsub, NK).
 __global__ void __launch_bounds__(256) k_cg_sub(State S, const cplx<double>* __restrict__ zu, int ib, Src src,
                                                 cplx<double>* out, const cplx<double>* __restrict__ other,
+                                                const cplx<double>* __restrict__ x, const cplx<double>* __restrict__ P,
                                                 int role, int it, int ncg) {
   const int k = blockIdx.y;
-  if (role != SUB_START && S.done[k]) return;
-  const int c = blockIdx.x;
+  const int skip = role != SUB_START ? S.done[k] : 0;
+  const int c = blockIdx.x, lane = threadIdx.x & (kWave - 1), wv = threadIdx.x / kWave;
   const size_t off = (size_t)k * S.NL;
   const double xhx = S.sc[k * kNS + XHX];
   const cplx<double>* B = zu + (size_t)k * S.NB * S.NL;
   const cplx<double>* zs = S.zs + (size_t)k * S.NB;
-  double v[1] = {0.0};
-#pragma unroll
-  for (int i = 0; i < kSubPPT; ++i) {
-    const int p = c * kSubChunk + i * 256 + threadIdx.x;
-    if (p < S.NL) {
-      cplx<double> e = src.at(k, S.NL, p, xhx);
+  const int p = c * kSubPts + lane, pc = min(p, S.NL - 1);
+  const bool dir = role != SUB_START && role != SUB_NONE;
+  cplx<double> e{0, 0}, o{0, 0}, xp{0, 0}, q{0, 0};
+  if (wv == 0) {
+    e = src.at(k, S.NL, pc, xhx);
+    if (role == SUB_PCDIR) o = other[off + pc];
+    if (dir) xp = x[off + pc];
+    if (dir && it > 1 && role != SUB_LEARN) q = P[off + pc];
+  }
 #pragma unroll 8
-      for (int j = 0; j < ib; ++j) {
-        const cplx<double> b = B[(size_t)j * S.NL + p], z = zs[j];
-        e.re -= b.re * z.re - b.im * z.im;
-        e.im -= b.re * z.im + b.im * z.re;
-      }
-      out[off + p] = e;
-      if (role == SUB_PCDIR) {
-        const cplx<double> o = other[off + p];
-        v[0] += e.re * o.re + e.im * o.im;
-      } else {
-        v[0] += e.re * e.re + e.im * e.im;
-      }
+  for (int j = wv; j < ib; j += 4) {
+    const cplx<double> b = B[(size_t)j * S.NL + pc], z = zs[j];
+    e.re -= b.re * z.re - b.im * z.im;
+    e.im -= b.re * z.im + b.im * z.re;
+  }
+  loaded(e);
+  if (skip) return;
+  __shared__ cplx<double> sh[3][kWave];
+  if (wv > 0) sh[wv - 1][lane] = e;
+  __syncthreads();
+  double v[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+  if (wv == 0 && p < S.NL) {
+#pragma unroll
+    for (int w = 0; w < 3; ++w) {
+      e.re += sh[w][lane].re;
+      e.im += sh[w][lane].im;
     }
+    out[off + p] = e;
+    v[0] = role == SUB_PCDIR ? e.re * o.re + e.im * o.im : e.re * e.re + e.im * e.im;
+    v[1] = xp.re * e.re + xp.im * e.im;
+    v[2] = xp.re * e.im - xp.im * e.re;
+    v[3] = xp.re * q.re + xp.im * q.im;
+    v[4] = xp.re * q.im - xp.im * q.re;
   }
   if (role == SUB_NONE) return;
-  if (role == SUB_LEARN) {
-    if (c == 0 && threadIdx.x == 0) S.sc[k * kNS + UK] = 0.0;
-    return;
-  }
-  double tot[1];
-  if (!last_block_sum<1>(v, S, S.nsub, c, tot)) return;
+  double tot[5];
+  if (!last_block_sum<5>(v, S, S.nsub, c, tot)) return;
   if (threadIdx.x != 0) return;
   double* sc = S.sc + k * kNS;
   if (role == SUB_START) {
     sc[SN] = 1.0 / sqrt(tot[0] * S.Hxyz);
     S.done[k] = 0;
     S.iters[(size_t)k * S.NB + ib] = ncg;
-  } else {
+    return;
+  }
+  double uk = 0.0;
+  if (role != SUB_LEARN) {
     const double s = tot[0] * S.Hxyz;
-    sc[UK] = it == 1 ? 0.0 : s / sc[GKGK];
+    if (it > 1) uk = s / sc[GKGK];
     sc[GKGK] = s;
   }
+  sc[UK] = uk;
+  sc[ZSR] = (uk != 0.0 ? tot[1] + uk * tot[3] : tot[1]) * S.Hxyz;
+  sc[ZSI] = (uk != 0.0 ? tot[2] + uk * tot[4] : tot[2]) * S.Hxyz;
 }
 
-// v *= SN (normalisation, CG.f90:72-73,104-105); also copies into dst when given.
-__global__ void __launch_bounds__(256) k_cg_scale(State S, cplx<double>* __restrict__ v, cplx<double>* __restrict__ dst,
-                                                  size_t dst_stride, int check_done) {
-  const int k = blockIdx.y;
-  if (check_done && S.done[k]) return;
-  const double s = S.sc[k * kNS + SN];
-  const size_t off = (size_t)k * S.NL;
-#pragma unroll
-  for (int i = 0; i < kPPT; ++i) {
-    const int p = blockIdx.x * kChunk + i * 256 + threadIdx.x;
-    if (p < S.NL) {
-      cplx<double> e = v[off + p];
-      e.re *= s;
-      e.im *= s;
-      v[off + p] = e;
-      if (dst) dst[(size_t)k * dst_stride + p] = e;
-    }
-  }
-}
-
-// Reductions of the form sum conj(a) b over the chunk; NQ = 1 takes the real
-// part, NQ = 2 the complex value.
-template <int NQ>
-__device__ __forceinline__ void dot_acc(double (&v)[NQ], cplx<double> a, cplx<double> b) {
-  v[0] += a.re * b.re + a.im * b.im;
-  if constexpr (NQ > 1) v[1] += a.re * b.im - a.im * b.re;
-}
-
-// xkHxk, xkTxk of the start vector (CG.f90:79-80).
-__global__ void __launch_bounds__(256) k_cg_xhx(State S, const cplx<double>* __restrict__ x,
-                                                const cplx<double>* __restrict__ hx, const cplx<double>* __restrict__ tx) {
-  const int k = blockIdx.y, c = blockIdx.x;
-  const size_t off = (size_t)k * S.NL;
-  double v[2] = {0.0, 0.0};
-#pragma unroll
-  for (int i = 0; i < kPPT; ++i) {
-    const int p = c * kChunk + i * 256 + threadIdx.x;
-    if (p < S.NL) {
-      const cplx<double> e = x[off + p], h = hx[off + p], t = tx[off + p];
-      v[0] += e.re * h.re + e.im * h.im;
-      v[1] += e.re * t.re + e.im * t.im;
-    }
-  }
-  double tot[2];
-  if (!last_block_sum<2>(v, S, S.nchunk, c, tot)) return;
-  if (threadIdx.x == 0) {
-    S.sc[k * kNS + XHX] = tot[0] * S.Hxyz;
-    S.sc[k * kNS + XTX] = tot[1] * S.Hxyz;
-  }
-}
-
-// p = dir + uk p (CG.f90:92-98), then zs = <x|p> Hxyz (CG.f90:103).
-__global__ void __launch_bounds__(256) k_cg_pupd(State S, const cplx<double>* __restrict__ dir,
-                                                 cplx<double>* __restrict__ P, const cplx<double>* __restrict__ x) {
-  const int k = blockIdx.y, c = blockIdx.x;
-  if (S.done[k]) return;
-  const size_t off = (size_t)k * S.NL;
-  const double uk = S.sc[k * kNS + UK];
-  double v[2] = {0.0, 0.0};
-#pragma unroll
-  for (int i = 0; i < kPPT; ++i) {
-    const int p = c * kChunk + i * 256 + threadIdx.x;
-    if (p < S.NL) {
-      cplx<double> d = dir[off + p];
-      if (uk != 0.0) {
-        const cplx<double> q = P[off + p];
-        d.re += uk * q.re;
-        d.im += uk * q.im;
-      }
-      P[off + p] = d;
-      dot_acc<2>(v, x[off + p], d);
-    }
-  }
-  double tot[2];
-  if (!last_block_sum<2>(v, S, S.nchunk, c, tot)) return;
-  if (threadIdx.x == 0) {
-    S.sc[k * kNS + ZSR] = tot[0] * S.Hxyz;
-    S.sc[k * kNS + ZSI] = tot[1] * S.Hxyz;
-  }
-}
-
-// pko = p - x zs, SN = 1/sqrt(|pko|^2 Hxyz) (CG.f90:103-105).
-__global__ void __launch_bounds__(256) k_cg_pko(State S, const cplx<double>* __restrict__ P,
+// p = d + uk p (CG.f90:92-98), o = p - x zs, SN = 1/sqrt(|o|^2 Hxyz)
+// (CG.f90:103-105).  o stays as it is: the H application and the rotation take
+// SN with it.  Grid (nvec, NK).
+__global__ void __launch_bounds__(256) k_cg_pko(State S, const cplx<double>* __restrict__ d, cplx<double>* __restrict__ P,
                                                 const cplx<double>* __restrict__ x, cplx<double>* __restrict__ pko) {
   const int k = blockIdx.y, c = blockIdx.x;
-  if (S.done[k]) return;
-  const size_t off = (size_t)k * S.NL;
-  const cplx<double> z{S.sc[k * kNS + ZSR], S.sc[k * kNS + ZSI]};
+  const int skip = S.done[k];
+  const double* sc = S.sc + k * kNS;
+  const double uk = sc[UK];
+  const cplx<double> z{sc[ZSR], sc[ZSI]};
+  const int p = c * 256 + threadIdx.x;
+  const size_t i = (size_t)k * S.NL + min(p, S.NL - 1);
+  const cplx<double> e = x[i], b = P[i];  // (P holds no numbers yet at uk = 0)
+  cplx<double> q = d[i];
+  loaded(e);
+  loaded(b);
+  loaded(q);
+  if (skip) return;
   double v[1] = {0.0};
-#pragma unroll
-  for (int i = 0; i < kPPT; ++i) {
-    const int p = c * kChunk + i * 256 + threadIdx.x;
-    if (p < S.NL) {
-      const cplx<double> e = x[off + p], q = P[off + p];
-      cplx<double> o;
-      o.re = q.re - (e.re * z.re - e.im * z.im);
-      o.im = q.im - (e.re * z.im + e.im * z.re);
-      pko[off + p] = o;
-      v[0] += o.re * o.re + o.im * o.im;
+  if (p < S.NL) {
+    if (uk != 0.0) {
+      q.re += uk * b.re;
+      q.im += uk * b.im;
     }
+    P[i] = q;
+    q.re -= e.re * z.re - e.im * z.im;
+    q.im -= e.re * z.im + e.im * z.re;
+    pko[i] = q;
+    v[0] = q.re * q.re + q.im * q.im;
   }
   double tot[1];
-  if (!last_block_sum<1>(v, S, S.nchunk, c, tot)) return;
+  if (!last_block_sum<1>(v, S, S.nvec, c, tot)) return;
   if (threadIdx.x == 0) S.sc[k * kNS + SN] = 1.0 / sqrt(tot[0] * S.Hxyz);
 }
 
-// 2x2 Rayleigh-Ritz of span{x, pko} (CG.f90:107-114).
-__global__ void __launch_bounds__(256) k_cg_rr(State S, const cplx<double>* __restrict__ x,
-                                               const cplx<double>* __restrict__ pko, const cplx<double>* __restrict__ hp,
-                                               int ib, int it) {
-  const int k = blockIdx.y, c = blockIdx.x;
-  if (S.done[k]) return;
-  const size_t off = (size_t)k * S.NL;
-  double v[3] = {0.0, 0.0, 0.0};
+// KB projections of the CG's vector and the term each sphere point adds
+// (pseudo_pt, ARTED/common/hpsi.f90:183-206), an atom per block:
+//   U(l) = Hxyz iuV(l) sum_j uV(j,l) e^{ik.r_j} v(J_j),  dps(j) = e^{-ik.r_j} sum_l uV(j,l) U(l)
+// so that the stencil pass reads one term per sphere point instead of four
+// projectors' tables and a sincos each: the two launches took 15 and 6 us on
+// 32^3 with 27 atoms.  A wave per projector, then a thread per point.  Grid (NI, NK).
+__global__ void __launch_bounds__(256) k_cg_kb(State S, const cplx<double>* __restrict__ in, KBTables kb,
+                                               const cplx<double>* __restrict__ ph, cplx<double>* __restrict__ dps,
+                                               int check_done) {
+  const int a = blockIdx.x, k = blockIdx.y;
+  const int skip = check_done ? S.done[k] : 0;
+  const int lane = threadIdx.x & (kWave - 1), wv = threadIdx.x / kWave;
+  const int j0 = kb.atom_start[a], m = kb.atom_start[a + 1] - j0;
+  const cplx<double>* E = in + (size_t)k * S.NL;
+  const cplx<double>* pk = ph + (size_t)k * kb.NPI + j0;
+  cplx<double>* dk = dps + (size_t)k * kb.NPI + j0;
+  constexpr int kPass = 16;
+  __shared__ cplx<double> U[kPass];
+  const int lb = kb.atom_lma[a], le = kb.atom_lma[a + 1];
+  for (int l0 = lb; l0 < le; l0 += kPass) {
+    const int nl = min(kPass, le - l0);
+    for (int l = wv; l < nl; l += 4) {
+      const double* uv = kb.uv + (size_t)(l0 + l) * kb.Nps;
+      double sr = 0.0, si = 0.0;
+      // three chunks with their loads in flight; indices past the sphere: its first point, weight zero
+      for (int jb = 0; jb < m; jb += 3 * kWave) {
+        cplx<double> e[3], f[3];
+        double u[3];
 #pragma unroll
-  for (int i = 0; i < kPPT; ++i) {
-    const int p = c * kChunk + i * 256 + threadIdx.x;
-    if (p < S.NL) {
-      const cplx<double> e = x[off + p], q = pko[off + p], h = hp[off + p];
-      v[0] += e.re * h.re + e.im * h.im;
-      v[1] += e.re * h.im - e.im * h.re;
-      v[2] += q.re * h.re + q.im * h.im;
+        for (int h = 0; h < 3; ++h) {
+          const int j = jb + h * kWave + lane, jc = j < m ? j : 0;
+          e[h] = E[kb.pidx[j0 + jc]];
+          f[h] = pk[jc];
+          u[h] = uv[jc];
+          u[h] = j < m ? u[h] : 0.0;
+        }
+#pragma unroll
+        for (int h = 0; h < 3; ++h) {
+          sr += u[h] * (f[h].re * e[h].re - f[h].im * e[h].im);
+          si += u[h] * (f[h].re * e[h].im + f[h].im * e[h].re);
+        }
+      }
+      sr = wave_sum(sr);
+      si = wave_sum(si);
+      const double f = S.Hxyz * kb.lma_sign[l0 + l];
+      if (lane == 0) U[l] = cplx<double>{sr * f, si * f};
     }
-  }
-  double tot[3];
-  if (!last_block_sum<3>(v, S, S.nchunk, c, tot)) return;
-  if (threadIdx.x != 0) return;
-  double* sc = S.sc + k * kNS;
-  const double xhx = sc[XHX];
-  const double xhp_r = tot[0] * S.Hxyz, xhp_i = tot[1] * S.Hxyz, php = tot[2] * S.Hxyz;
-  const double a2 = xhp_r * xhp_r + xhp_i * xhp_i;
-  const double ev = 0.5 * ((xhx + php) - sqrt((xhx - php) * (xhx - php) + 4.0 * a2));
-  double cxr = xhp_r / (ev - xhx), cxi = xhp_i / (ev - xhx);
-  const double cp = 1.0 / sqrt(1.0 + (cxr * cxr + cxi * cxi));
-  cxr *= cp;
-  cxi *= cp;
-  sc[EVX] = ev;
-  sc[CXR] = cxr;
-  sc[CXI] = cxi;
-  sc[CP] = cp;
-  if (fabs(ev - xhx) < 1e-15) {
-    S.done[k] = 1;
-    S.iters[(size_t)k * S.NB + ib] = it;
+    __syncthreads();
+    if (skip) return;
+    for (int j = threadIdx.x; j < m; j += 256) {
+      cplx<double> t{0, 0};
+      for (int l = 0; l < nl; ++l) {
+        const double u = kb.uv[(size_t)(l0 + l) * kb.Nps + j];
+        t.re += u * U[l].re;
+        t.im += u * U[l].im;
+      }
+      const cplx<double> f = pk[j];
+      cplx<double> r{f.re * t.re + f.im * t.im, f.re * t.im - f.im * t.re};  // conj(f) t
+      if (l0 > lb) {
+        r.re += dk[j].re;
+        r.im += dk[j].im;
+      }
+      dk[j] = r;
+    }
+    __syncthreads();
   }
 }
 
-// x = cx x + cp pko, hx, tx likewise (CG.f90:115-117); then <x|H|x>, <x|T|x>
-// (CG.f90:118-119).
+// What an H application of the CG ends with.
+enum : int {
+  H_START = 0,  // start vector: x = s v; <x|H|x>, <x|T|x> (CG.f90:79-80), |x|^2
+  H_RR = 1,     // search direction q = s o: 2x2 Rayleigh-Ritz of span{x, q} (CG.f90:107-114)
+  H_EFIN = 2    // stored band = s x: e = <x|H|x> (CG.f90:122-125)
+};
+
+// h = s H v, t = s T v (nullable: only the kinetic preconditioner reads <x|T|x>)
+// of the vector v, s = 1/|v|, with the KB terms of k_cg_kb; the scaled vector
+// itself for H_START and H_EFIN; then the role's sums, whose operands it has at
+// hand.  Grid (nvec, NK).
+template <int ROLE>
+__global__ void __launch_bounds__(256) k_cg_h(State S, const cplx<double>* __restrict__ v, const double* __restrict__ kac,
+                                              const double* __restrict__ vloc, Grid g, KBTables kb,
+                                              const cplx<double>* __restrict__ dps, cplx<double>* __restrict__ hv,
+                                              cplx<double>* __restrict__ tv, cplx<double>* __restrict__ xo, size_t xstride,
+                                              const cplx<double>* __restrict__ x, int ib, int it) {
+  const int k = blockIdx.y, c = blockIdx.x;
+  const int skip = ROLE == H_RR ? S.done[k] : 0;
+  double* sc = S.sc + k * kNS;
+  const int p = c * 256 + threadIdx.x;
+  const double s = sc[ROLE == H_EFIN ? XN : SN];
+  double sum[3] = {0.0, 0.0, 0.0};
+  if (p < S.NL) {
+    const size_t i = (size_t)k * S.NL + p;
+    const int tp = kb.pt2t[p];
+    cplx<double> xp{0, 0};
+    if (ROLE == H_RR) xp = x[i];
+    double kx, ky, kz;
+    orbital_k(kac, S.NK, k, 0, 0, 0, kx, ky, kz);
+    cplx<double> e, t;
+    double V;
+    cplx<double> f = stencil_point<double>(v + (size_t)k * S.NL, p, kx, ky, kz, vloc, g, e, V);
+    loaded(f);
+    loaded(xp);
+    if (ROLE == H_RR && skip) return;  // (of all threads of the block: one k)
+    if (tv) t = cplx<double>{f.re - V * e.re, f.im - V * e.im};
+    if (tp >= 0) {
+      const cplx<double>* d = dps + (size_t)k * kb.NPI;
+      for (int q = kb.tj_start[tp]; q < kb.tj_start[tp + 1]; ++q) {
+        const cplx<double> a = d[kb.tj[q]];
+        f.re += a.re;
+        f.im += a.im;
+      }
+    }
+    f.re *= s;
+    f.im *= s;
+    e.re *= s;
+    e.im *= s;
+    hv[i] = f;
+    if (ROLE != H_RR) xo[(size_t)k * xstride + p] = e;
+    if (tv) {
+      t.re *= s;
+      t.im *= s;
+      tv[i] = t;
+    }
+    if (ROLE == H_RR) {
+      sum[0] = xp.re * f.re + xp.im * f.im;
+      sum[1] = xp.re * f.im - xp.im * f.re;
+      sum[2] = e.re * f.re + e.im * f.im;
+    } else {
+      sum[0] = e.re * f.re + e.im * f.im;
+      if (ROLE == H_START) {
+        if (tv) sum[1] = e.re * t.re + e.im * t.im;
+        sum[2] = e.re * e.re + e.im * e.im;
+      }
+    }
+  }
+  double tot[3];
+  if (!last_block_sum<3>(sum, S, S.nvec, c, tot)) return;
+  if (threadIdx.x != 0) return;
+  if (ROLE == H_EFIN) {
+    sc[EFIN] = tot[0] * S.Hxyz;
+  } else if (ROLE == H_START) {
+    sc[XHX] = tot[0] * S.Hxyz;
+    sc[XTX] = tot[1] * S.Hxyz;
+    sc[XN] = 1.0 / sqrt(tot[2] * S.Hxyz);
+  } else {
+    const double xhx = sc[XHX];
+    const double xhp_r = tot[0] * S.Hxyz, xhp_i = tot[1] * S.Hxyz, php = tot[2] * S.Hxyz;
+    const double a2 = xhp_r * xhp_r + xhp_i * xhp_i;
+    const double ev = 0.5 * ((xhx + php) - sqrt((xhx - php) * (xhx - php) + 4.0 * a2));
+    double cxr = xhp_r / (ev - xhx), cxi = xhp_i / (ev - xhx);
+    const double cp = 1.0 / sqrt(1.0 + (cxr * cxr + cxi * cxi));
+    cxr *= cp;
+    cxi *= cp;
+    sc[EVX] = ev;
+    sc[CXR] = cxr;
+    sc[CXI] = cxi;
+    sc[CP] = cp;
+    if (fabs(ev - xhx) < 1e-15) {
+      S.done[k] = 1;
+      S.iters[(size_t)k * S.NB + ib] = it;
+    }
+  }
+}
+
+// x = cx x + cp q, q = SN pko; hx and (nullable) tx likewise (CG.f90:115-117);
+// then <x|H|x>, <x|T|x> (CG.f90:118-119) and 1/|x| for the stored band
+// (CG.f90:122).  Grid (nvec, NK).
 __global__ void __launch_bounds__(256) k_cg_rotate(State S, cplx<double>* __restrict__ x, cplx<double>* __restrict__ hx,
                                                    cplx<double>* __restrict__ tx, const cplx<double>* __restrict__ pko,
                                                    const cplx<double>* __restrict__ hp, const cplx<double>* __restrict__ tp) {
   const int k = blockIdx.y, c = blockIdx.x;
-  if (S.done[k]) return;
-  const size_t off = (size_t)k * S.NL;
+  const int skip = S.done[k];
   const double* sc = S.sc + k * kNS;
   const cplx<double> cx{sc[CXR], sc[CXI]};
-  const double cp = sc[CP];
-  double v[2] = {0.0, 0.0};
-#pragma unroll
-  for (int i = 0; i < kPPT; ++i) {
-    const int p = c * kChunk + i * 256 + threadIdx.x;
-    if (p < S.NL) {
-      cplx<double> e = cmulc(cx, x[off + p]), h = cmulc(cx, hx[off + p]), t = cmulc(cx, tx[off + p]);
-      const cplx<double> q = pko[off + p], hq = hp[off + p], tq = tp[off + p];
-      e.re += cp * q.re;
-      e.im += cp * q.im;
-      h.re += cp * hq.re;
-      h.im += cp * hq.im;
+  const double cp = sc[CP], sn = sc[SN];
+  const int p = c * 256 + threadIdx.x;
+  const size_t i = (size_t)k * S.NL + min(p, S.NL - 1);
+  cplx<double> e = x[i], h = hx[i];
+  const cplx<double> q = pko[i], hq = hp[i];
+  loaded(e);
+  loaded(h);
+  loaded(q);
+  loaded(hq);
+  if (skip) return;
+  double v[3] = {0.0, 0.0, 0.0};
+  if (p < S.NL) {
+    e = cmulc(cx, e);
+    h = cmulc(cx, h);
+    e.re += cp * (sn * q.re);
+    e.im += cp * (sn * q.im);
+    h.re += cp * hq.re;
+    h.im += cp * hq.im;
+    x[i] = e;
+    hx[i] = h;
+    v[0] = e.re * h.re + e.im * h.im;
+    v[2] = e.re * e.re + e.im * e.im;
+    if (tx) {
+      cplx<double> t = cmulc(cx, tx[i]);
+      const cplx<double> tq = tp[i];
       t.re += cp * tq.re;
       t.im += cp * tq.im;
-      x[off + p] = e;
-      hx[off + p] = h;
-      tx[off + p] = t;
-      v[0] += e.re * h.re + e.im * h.im;
-      v[1] += e.re * t.re + e.im * t.im;
+      tx[i] = t;
+      v[1] = e.re * t.re + e.im * t.im;
     }
   }
-  double tot[2];
-  if (!last_block_sum<2>(v, S, S.nchunk, c, tot)) return;
+  double tot[3];
+  if (!last_block_sum<3>(v, S, S.nvec, c, tot)) return;
   if (threadIdx.x == 0) {
     S.sc[k * kNS + XHX] = tot[0] * S.Hxyz;
     S.sc[k * kNS + XTX] = tot[1] * S.Hxyz;
+    S.sc[k * kNS + XN] = 1.0 / sqrt(tot[2] * S.Hxyz);
   }
 }
 
-// Final normalisation factor of the band (CG.f90:122).
-__global__ void __launch_bounds__(256) k_cg_norm(State S, const cplx<double>* __restrict__ x) {
-  const int k = blockIdx.y, c = blockIdx.x;
-  const size_t off = (size_t)k * S.NL;
-  double v[1] = {0.0};
-#pragma unroll
-  for (int i = 0; i < kPPT; ++i) {
-    const int p = c * kChunk + i * 256 + threadIdx.x;
-    if (p < S.NL) {
-      const cplx<double> e = x[off + p];
-      v[0] += e.re * e.re + e.im * e.im;
-    }
-  }
-  double tot[1];
-  if (!last_block_sum<1>(v, S, S.nchunk, c, tot)) return;
-  if (threadIdx.x == 0) S.sc[k * kNS + SN] = 1.0 / sqrt(tot[0] * S.Hxyz);
-}
-
-// e = <x|Hx> Hxyz of the stored band (CG.f90:125).
-__global__ void __launch_bounds__(256) k_cg_efin(State S, const cplx<double>* __restrict__ x,
-                                                 const cplx<double>* __restrict__ hp) {
-  const int k = blockIdx.y, c = blockIdx.x;
-  const size_t off = (size_t)k * S.NL;
-  double v[1] = {0.0};
-#pragma unroll
-  for (int i = 0; i < kPPT; ++i) {
-    const int p = c * kChunk + i * 256 + threadIdx.x;
-    if (p < S.NL) dot_acc<1>(v, x[off + p], hp[off + p]);
-  }
-  double tot[1];
-  if (!last_block_sum<1>(v, S, S.nchunk, c, tot)) return;
-  if (threadIdx.x == 0) S.sc[k * kNS + EFIN] = tot[0] * S.Hxyz;
-}
-
-// esp_var(ib,k) = sqrt(|Hx - e x|^2 Hxyz) occ(ib,k) (CG.f90:126).
-__global__ void __launch_bounds__(256) k_cg_resid(State S, const cplx<double>* __restrict__ x,
+// esp_var(ib,k) = sqrt(|Hx - e x|^2 Hxyz) occ(ib,k) of the stored band x
+// (CG.f90:126).  Grid (nvec, NK).
+__global__ void __launch_bounds__(256) k_cg_resid(State S, const cplx<double>* __restrict__ x, size_t xstride,
                                                   const cplx<double>* __restrict__ hp, int ib) {
   const int k = blockIdx.y, c = blockIdx.x;
-  const size_t off = (size_t)k * S.NL;
   const double e = S.sc[k * kNS + EFIN];
+  const int p = c * 256 + threadIdx.x;
   double v[1] = {0.0};
-#pragma unroll
-  for (int i = 0; i < kPPT; ++i) {
-    const int p = c * kChunk + i * 256 + threadIdx.x;
-    if (p < S.NL) {
-      const cplx<double> a = x[off + p], h = hp[off + p];
-      const double r = h.re - e * a.re, q = h.im - e * a.im;
-      v[0] += r * r + q * q;
-    }
+  if (p < S.NL) {
+    const cplx<double> a = x[(size_t)k * xstride + p], h = hp[(size_t)k * S.NL + p];
+    const double r = h.re - e * a.re, q = h.im - e * a.im;
+    v[0] = r * r + q * q;
   }
   double tot[1];
-  if (!last_block_sum<1>(v, S, S.nchunk, c, tot)) return;
+  if (!last_block_sum<1>(v, S, S.nvec, c, tot)) return;
   if (threadIdx.x == 0) {
     const size_t o = (size_t)k * S.NB + ib;
     S.esp_var[o] = sqrt(tot[0] * S.Hxyz) * S.occ[o];
@@ -765,46 +855,40 @@ __global__ void __launch_bounds__(256) k_rotate_bands(const cplx<double>* __rest
 
 // Gram-Schmidt step of band ib in place (Gram_Schmidt_ompk,
 // ARTED/GS/Gram_Schmidt.f90:43-50): v -= sum_{j<ib} zs_j B_j; with_norm ends
-// with SN = 1/sqrt(|v|^2 Hxyz).  Grid (nsub, NK).
+// with SN = 1/sqrt(|v|^2 Hxyz).  Grid (nvec, NK).
 __global__ void __launch_bounds__(256) k_gs_sub(State S, cplx<double>* __restrict__ zu, int ib, int with_norm) {
   const int k = blockIdx.y, c = blockIdx.x;
   cplx<double>* B = zu + (size_t)k * S.NB * S.NL;
   cplx<double>* v = B + (size_t)ib * S.NL;
   const cplx<double>* zs = S.zs + (size_t)k * S.NB;
+  const int p = c * 256 + threadIdx.x;
   double a[1] = {0.0};
-#pragma unroll
-  for (int i = 0; i < kSubPPT; ++i) {
-    const int p = c * kSubChunk + i * 256 + threadIdx.x;
-    if (p < S.NL) {
-      cplx<double> e = v[p];
+  if (p < S.NL) {
+    cplx<double> e = v[p];
 #pragma unroll 8
-      for (int j = 0; j < ib; ++j) {
-        const cplx<double> b = B[(size_t)j * S.NL + p], z = zs[j];
-        e.re -= b.re * z.re - b.im * z.im;
-        e.im -= b.re * z.im + b.im * z.re;
-      }
-      v[p] = e;
-      a[0] += e.re * e.re + e.im * e.im;
+    for (int j = 0; j < ib; ++j) {
+      const cplx<double> b = B[(size_t)j * S.NL + p], z = zs[j];
+      e.re -= b.re * z.re - b.im * z.im;
+      e.im -= b.re * z.im + b.im * z.re;
     }
+    v[p] = e;
+    a[0] = e.re * e.re + e.im * e.im;
   }
   if (!with_norm) return;
   double tot[1];
-  if (!last_block_sum<1>(a, S, S.nsub, c, tot)) return;
+  if (!last_block_sum<1>(a, S, S.nvec, c, tot)) return;
   if (threadIdx.x == 0) S.sc[k * kNS + SN] = 1.0 / sqrt(tot[0] * S.Hxyz);
 }
 
-// band ib *= SN.  Grid (nchunk, NK).
+// band ib *= SN.  Grid (nvec, NK).
 __global__ void __launch_bounds__(256) k_gs_scale(State S, cplx<double>* __restrict__ zu, int ib) {
   const int k = blockIdx.y;
   const double f = S.sc[k * kNS + SN];
   cplx<double>* v = zu + ((size_t)k * S.NB + ib) * S.NL;
-#pragma unroll
-  for (int i = 0; i < kPPT; ++i) {
-    const int p = blockIdx.x * kChunk + i * 256 + threadIdx.x;
-    if (p < S.NL) {
-      v[p].re *= f;
-      v[p].im *= f;
-    }
+  const int p = blockIdx.x * 256 + threadIdx.x;
+  if (p < S.NL) {
+    v[p].re *= f;
+    v[p].im *= f;
   }
 }
 

@@ -39,6 +39,8 @@ struct KBTables {
   const int* t_start;     // (NT+1) first entry of each touched point
   const int* e_lma;       // (NE) projector of each entry
   const int* e_jp;        // (NE) packed point of each entry
+  const int* tj_start;    // (NT+1) first packed point of each touched point
+  const int* tj;          // the touched points' packed points, of atoms with projectors
 };
 
 constexpr int kWave = 64;
@@ -197,6 +199,17 @@ __device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
   __builtin_amdgcn_s_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// Values handed from one block to another within a launch: agent-scope atomic
+// stores and loads, which go past the caches that other compute units do not
+// share, and a wait for the stores (acknowledged once they are visible there)
+// before the wave, or after a barrier its block, arrives at a counter with a
+// relaxed add.  Release and acquire on that add would write back and invalidate
+// the L2 caches in every block, and only data stored in other ways needs that.
+__device__ __forceinline__ void agent_stores_done() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+__device__ __forceinline__ unsigned agent_arrive(unsigned* c) {
+  return __hip_atomic_fetch_add(c, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 __device__ __forceinline__ void sincos_t(double x, double* s, double* c) { sincos(x, s, c); }

@@ -19,10 +19,11 @@ struct PcInfer {
 };
 
 struct GsState {
-  int NK = 0, NB = 0, NL = 0, Nlma = 0, nchunk = 0, ngroup = 0;
+  int NK = 0, NB = 0, NL = 0, Nlma = 0, NPI = 0, nchunk = 0, ngroup = 0;
   std::vector<void*> bufs;
   cplx<double>* w[11] = {};  // X HX TX G P PKO HP TP KG T1 T2, NK*NL each
-  void* uv = nullptr;        // NK*Nlma
+  cplx<double>* ph = nullptr;   // (NK, NPI) phases of the sphere points at the CG's k
+  cplx<double>* dps = nullptr;  // (NK, NPI) KB term of each
   double* sc = nullptr;
   int* done = nullptr;
   int* iters = nullptr;
@@ -122,7 +123,7 @@ static void kinetic_tables(const Grid& g, std::vector<double>& tw, std::vector<d
 
 static int gs_ensure(salmon_ctx* c) {
   GsState* s = (GsState*)c->gs;
-  if (s && s->NK == c->NK && s->NB == c->NB && s->Nlma == c->kb.Nlma) return SALMON_OK;
+  if (s && s->NK == c->NK && s->NB == c->NB && s->Nlma == c->kb.Nlma && s->NPI == c->kb.NPI) return SALMON_OK;
   gs_free(c);
   s = new GsState();
   c->gs = s;
@@ -130,14 +131,16 @@ static int gs_ensure(salmon_ctx* c) {
   s->NB = c->NB;
   s->NL = c->g.NL;
   s->Nlma = c->kb.Nlma;
+  s->NPI = c->kb.NPI;
   s->nchunk = (s->NL + kChunk - 1) / kChunk;
   s->ngroup = (s->NB + kJG - 1) / kJG;
-  s->pstride = std::max(s->nchunk * s->ngroup * kPartQ, (s->NL + kSubChunk - 1) / kSubChunk);
+  s->pstride = std::max(s->nchunk * s->ngroup * kPartQ, (s->NL + kSubPts - 1) / kSubPts * 5);
   const size_t nv = (size_t)s->NK * s->NL;
   int r;
   for (int i = 0; i < 11; ++i)
     if ((r = gs_alloc(c, s, &s->w[i], nv))) return r;
-  if ((r = gs_alloc(c, s, (cplx<double>**)&s->uv, (size_t)s->NK * std::max(1, c->kb.Nlma)))) return r;
+  if ((r = gs_alloc(c, s, &s->ph, (size_t)s->NK * s->NPI))) return r;
+  if ((r = gs_alloc(c, s, &s->dps, (size_t)s->NK * s->NPI))) return r;
   if ((r = gs_alloc(c, s, &s->sc, (size_t)s->NK * kNS))) return r;
   if ((r = gs_alloc(c, s, &s->done, (size_t)s->NK))) return r;
   if ((r = gs_alloc(c, s, &s->iters, (size_t)s->NK * s->NB))) return r;
@@ -196,7 +199,8 @@ static State gs_view(salmon_ctx* c, GsState* s) {
   S.NB = s->NB;
   S.NL = s->NL;
   S.nchunk = s->nchunk;
-  S.nsub = (s->NL + kSubChunk - 1) / kSubChunk;
+  S.nsub = (s->NL + kSubPts - 1) / kSubPts;
+  S.nvec = (s->NL + 255) / 256;
   S.pstride = s->pstride;
   S.Hxyz = c->g.Hxyz;
   return S;
@@ -224,18 +228,42 @@ static int kinetic_apply(salmon_ctx* c, GsState* s, const State& S, const cplx<d
   return pass(t2, out, 2, +1, nullptr);
 }
 
-// CG_ompk over all bands of all k (FP64 orbitals).
+// CG_ompk over all bands of all k (FP64 orbitals).  An iteration is a chain of
+// launches each too short to hide its start and its reduction's end, so its
+// steps share launches where one's results are the next one's operands: nine
+// launches without a preconditioner became six (the scalings go with the H
+// application and the rotation, the 2x2 sums with the H application, the update
+// of the search direction with its orthogonalisation).
 static int cg_run(salmon_ctx* c, int ncg, int precond) {
   GsState* s = (GsState*)c->gs;
   State S = gs_view(c, s);
   cplx<double>* zu = (cplx<double>*)c->d_zu;
   cplx<double>** w = s->w;
   const int NK = s->NK, NB = s->NB, NL = s->NL;
-  const dim3 gv(s->nchunk, NK), blk(256), gsub(S.nsub, NK);
+  const dim3 gv(S.nvec, NK), blk(256), gsub(S.nsub, NK);
   const size_t bstride = (size_t)NB * NL;
+  const bool kinetic = precond == SALMON_PC_KINETIC;
+  cplx<double>*const tx = kinetic ? w[W_TX] : nullptr, *const tp = kinetic ? w[W_TP] : nullptr;
   int r;
-  auto H = [&](const cplx<double>* in, cplx<double>* out, cplx<double>* tt) {
-    return apply_h<double>(c, in, out, tt, 0, NK, 1, NK, c->d_kac, 0, 0, 0, s->uv);
+  if (c->kb.Nlma > 0) {
+    hipLaunchKernelGGL(k_phase_table<double>, dim3(((long)NK * c->kb.NPI + 255) / 256), blk, 0, c->stream,
+                       (const double*)c->d_kac, NK, 0.0, 0.0, 0.0, c->kb, s->ph);
+    LAUNCHCHK(c);
+  }
+  // H of the vector v; its scaled copy (H_START, H_EFIN) into xo
+  auto H = [&](auto role, const cplx<double>* v, cplx<double>* hv, cplx<double>* tv, cplx<double>* xo, size_t xstride,
+               int ib, int it) -> int {
+    constexpr int R = decltype(role)::value;
+    Region reg(c, SALMON_LOG_HPSI);
+    if (c->kb.Nlma > 0) {
+      hipLaunchKernelGGL(k_cg_kb, dim3(c->kb.NI, NK), blk, 0, c->stream, S, v, c->kb, (const cplx<double>*)s->ph, s->dps,
+                         R == H_RR ? 1 : 0);
+      LAUNCHCHK(c);
+    }
+    hipLaunchKernelGGL(k_cg_h<R>, gv, blk, 0, c->stream, S, v, (const double*)c->d_kac, (const double*)c->d_vloc, c->g,
+                       c->kb, (const cplx<double>*)s->dps, hv, tv, xo, xstride, (const cplx<double>*)w[W_X], ib, it);
+    LAUNCHCHK(c);
+    return SALMON_OK;
   };
   auto proj = [&](int ib, Src src, int mode, int check) -> int {
     if (ib == 0) return SALMON_OK;
@@ -244,26 +272,24 @@ static int cg_run(salmon_ctx* c, int ncg, int precond) {
     LAUNCHCHK(c);
     return SALMON_OK;
   };
+  auto sub = [&](int ib, Src src, cplx<double>* out, const cplx<double>* other, int role, int it) -> int {
+    hipLaunchKernelGGL(k_cg_sub, gsub, blk, 0, c->stream, S, (const cplx<double>*)zu, ib, src, out, other,
+                       (const cplx<double>*)w[W_X], (const cplx<double>*)w[W_P], role, it, ncg);
+    LAUNCHCHK(c);
+    return SALMON_OK;
+  };
   const Src resid{nullptr, 0, w[W_HX], w[W_X]};
   for (int ib = 0; ib < NB; ++ib) {
     const Src start{zu + (size_t)ib * NL, bstride, nullptr, nullptr};
     // start vector orthogonalised to the lower bands and normalised (CG.f90:67-74)
     if ((r = proj(ib, start, PROJ_START, 0))) return r;
-    hipLaunchKernelGGL(k_cg_sub, gsub, blk, 0, c->stream, S, (const cplx<double>*)zu, ib, start, w[W_X],
-                       (const cplx<double>*)nullptr, (int)SUB_START, 0, ncg);
-    LAUNCHCHK(c);
-    hipLaunchKernelGGL(k_cg_scale, gv, blk, 0, c->stream, S, w[W_X], (cplx<double>*)nullptr, (size_t)0, 0);
-    LAUNCHCHK(c);
-    if ((r = H(w[W_X], w[W_HX], w[W_TX]))) return r;
-    hipLaunchKernelGGL(k_cg_xhx, gv, blk, 0, c->stream, S, w[W_X], w[W_HX], w[W_TX]);
-    LAUNCHCHK(c);
+    if ((r = sub(ib, start, w[W_T1], nullptr, SUB_START, 0))) return r;
+    if ((r = H(std::integral_constant<int, H_START>(), w[W_T1], w[W_HX], tx, w[W_X], (size_t)NL, ib, 0))) return r;
     for (int it = 1; it <= ncg; ++it) {
       // residual orthogonalised to the lower bands (CG.f90:85-90)
       if ((r = proj(ib, resid, PROJ_VEC, 1))) return r;
       const cplx<double>* dir = w[W_G];
-      hipLaunchKernelGGL(k_cg_sub, gsub, blk, 0, c->stream, S, (const cplx<double>*)zu, ib, resid, w[W_G],
-                         (const cplx<double>*)nullptr, (int)(precond == SALMON_PC_NONE ? SUB_GRAD : SUB_NONE), it, ncg);
-      LAUNCHCHK(c);
+      if ((r = sub(ib, resid, w[W_G], nullptr, precond == SALMON_PC_NONE ? SUB_GRAD : SUB_NONE, it))) return r;
       if (s->recording && s->smp_n < s->smp_cap && NK == 1 && (s->smp_seen++ % s->smp_stride) == 0) {
         const int slot = s->smp_n++;
         hipLaunchKernelGGL(k_pc_record, dim3((NL + 255) / 256), blk, 0, c->stream, S, (const cplx<double>*)w[W_G],
@@ -279,40 +305,25 @@ static int cg_run(salmon_ctx* c, int ncg, int precond) {
         }
         const Src kg{w[W_KG], (size_t)NL, nullptr, nullptr};
         if ((r = proj(ib, kg, PROJ_VEC, 1))) return r;
-        hipLaunchKernelGGL(k_cg_sub, gsub, blk, 0, c->stream, S, (const cplx<double>*)zu, ib, kg, w[W_KG],
-                           (const cplx<double>*)w[W_G], (int)(precond == SALMON_PC_LEARNED ? SUB_LEARN : SUB_PCDIR),
-                           it, ncg);
-        LAUNCHCHK(c);
+        if ((r = sub(ib, kg, w[W_KG], w[W_G], precond == SALMON_PC_LEARNED ? SUB_LEARN : SUB_PCDIR, it))) return r;
         dir = w[W_KG];
       }
       // search direction, orthogonalised to x and normalised (CG.f90:92-106)
-      hipLaunchKernelGGL(k_cg_pupd, gv, blk, 0, c->stream, S, dir, w[W_P], (const cplx<double>*)w[W_X]);
+      hipLaunchKernelGGL(k_cg_pko, gv, blk, 0, c->stream, S, dir, w[W_P], (const cplx<double>*)w[W_X], w[W_PKO]);
       LAUNCHCHK(c);
-      hipLaunchKernelGGL(k_cg_pko, gv, blk, 0, c->stream, S, (const cplx<double>*)w[W_P], (const cplx<double>*)w[W_X],
-                         w[W_PKO]);
-      LAUNCHCHK(c);
-      hipLaunchKernelGGL(k_cg_scale, gv, blk, 0, c->stream, S, w[W_PKO], (cplx<double>*)nullptr, (size_t)0, 1);
-      LAUNCHCHK(c);
-      if ((r = H(w[W_PKO], w[W_HP], w[W_TP]))) return r;
-      // 2x2 Rayleigh-Ritz and the update (CG.f90:107-119)
-      hipLaunchKernelGGL(k_cg_rr, gv, blk, 0, c->stream, S, (const cplx<double>*)w[W_X], (const cplx<double>*)w[W_PKO],
-                         (const cplx<double>*)w[W_HP], ib, it);
-      LAUNCHCHK(c);
-      hipLaunchKernelGGL(k_cg_rotate, gv, blk, 0, c->stream, S, w[W_X], w[W_HX], w[W_TX],
-                         (const cplx<double>*)w[W_PKO], (const cplx<double>*)w[W_HP], (const cplx<double>*)w[W_TP]);
+      // its H, the 2x2 Rayleigh-Ritz and the update (CG.f90:107-119)
+      if ((r = H(std::integral_constant<int, H_RR>(), w[W_PKO], w[W_HP], tp, nullptr, 0, ib, it))) return r;
+      hipLaunchKernelGGL(k_cg_rotate, gv, blk, 0, c->stream, S, w[W_X], w[W_HX], tx, (const cplx<double>*)w[W_PKO],
+                         (const cplx<double>*)w[W_HP], (const cplx<double>*)tp);
       LAUNCHCHK(c);
     }
     // store the normalised band and its residual (CG.f90:122-126)
-    hipLaunchKernelGGL(k_cg_norm, gv, blk, 0, c->stream, S, (const cplx<double>*)w[W_X]);
-    LAUNCHCHK(c);
-    hipLaunchKernelGGL(k_cg_scale, gv, blk, 0, c->stream, S, w[W_X], zu + (size_t)ib * NL, bstride, 0);
-    LAUNCHCHK(c);
+    cplx<double>* band = zu + (size_t)ib * NL;
+    if ((r = H(std::integral_constant<int, H_EFIN>(), w[W_X], w[W_HP], nullptr, band, bstride, ib, 0))) return r;
     // row ib of the lower bands' Gram matrix, for the later bands' projections
-    if (ib + 1 < NB && (r = proj(ib, Src{zu + (size_t)ib * NL, bstride, nullptr, nullptr}, PROJ_GRAM, 0))) return r;
-    if ((r = H(w[W_X], w[W_HP], w[W_TP]))) return r;
-    hipLaunchKernelGGL(k_cg_efin, gv, blk, 0, c->stream, S, (const cplx<double>*)w[W_X], (const cplx<double>*)w[W_HP]);
-    LAUNCHCHK(c);
-    hipLaunchKernelGGL(k_cg_resid, gv, blk, 0, c->stream, S, (const cplx<double>*)w[W_X], (const cplx<double>*)w[W_HP], ib);
+    if (ib + 1 < NB && (r = proj(ib, Src{band, bstride, nullptr, nullptr}, PROJ_GRAM, 0))) return r;
+    hipLaunchKernelGGL(k_cg_resid, gv, blk, 0, c->stream, S, (const cplx<double>*)band, bstride,
+                       (const cplx<double>*)w[W_HP], ib);
     LAUNCHCHK(c);
   }
   return SALMON_OK;
@@ -328,18 +339,18 @@ static int gram_schmidt_multi(salmon_ctx* c, cplx<double>* zu) {
   if ((r = gs_ensure(c))) return r;
   GsState* s = (GsState*)c->gs;
   State S = gs_view(c, s);
-  const dim3 gv(s->nchunk, s->NK), blk(256), gsub(S.nsub, s->NK);
+  const dim3 gv(S.nvec, s->NK), blk(256);
   for (int ib = 0; ib < s->NB; ++ib) {
     const Src v{zu + (size_t)ib * s->NL, (size_t)s->NB * s->NL, nullptr, nullptr};
     for (int pass = 0; pass < 2 && ib > 0; ++pass) {
       hipLaunchKernelGGL(k_cg_proj, dim3(s->nchunk, (ib + kJG - 1) / kJG, s->NK), blk, 0, c->stream, S,
                          (const cplx<double>*)zu, ib, v, (int)PROJ_PLAIN, 0);
       LAUNCHCHK(c);
-      hipLaunchKernelGGL(k_gs_sub, gsub, blk, 0, c->stream, S, zu, ib, pass == 1 ? 1 : 0);
+      hipLaunchKernelGGL(k_gs_sub, gv, blk, 0, c->stream, S, zu, ib, pass == 1 ? 1 : 0);
       LAUNCHCHK(c);
     }
     if (ib == 0) {
-      hipLaunchKernelGGL(k_gs_sub, gsub, blk, 0, c->stream, S, zu, 0, 1);
+      hipLaunchKernelGGL(k_gs_sub, gv, blk, 0, c->stream, S, zu, 0, 1);
       LAUNCHCHK(c);
     }
     hipLaunchKernelGGL(k_gs_scale, gv, blk, 0, c->stream, S, zu, ib);

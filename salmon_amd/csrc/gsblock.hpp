@@ -59,18 +59,17 @@ __device__ __forceinline__ cplx<double> load_agent(const cplx<double>* p) {
 }
 
 // Whether this block is the last of n to arrive at *c (which returns to zero);
-// all of its threads get the answer, and the others' stores are visible to them.
+// all of its threads get the answer, and the others' store_agent values are visible to them.
 __device__ __forceinline__ bool arrive_last(unsigned* c, unsigned n) {
   __shared__ int last;
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");  // every wave's stores, not only the first's
+  agent_stores_done();  // every wave's
   __syncthreads();
   if (threadIdx.x == 0) {
-    last = __hip_atomic_fetch_add(c, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == n - 1;
+    last = agent_arrive(c) == n - 1;
     if (last) __hip_atomic_store(c, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
   __syncthreads();
   const bool l = last != 0;
-  if (l) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
   __syncthreads();
   return l;
 }

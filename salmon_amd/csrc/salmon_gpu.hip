@@ -1028,17 +1028,19 @@ int salmon_gpu_set_projectors(salmon_ctx* c, int NI, int Nps, const int* Mps, co
     const int a = lma_atom[l];
     for (int j = 0; j < Mps[a]; ++j) per[pidx[start[a] + j]].push_back({start[a] + j, l});
   }
-  std::vector<int> pt2t(g.NL, -1), tstart(1, 0), elma, ejp;
+  std::vector<int> pt2t(g.NL, -1), tstart(1, 0), elma, ejp, tjstart(1, 0), tj;
   int NT = 0;
   for (int p = 0; p < g.NL; ++p) {
     if (per[p].empty()) continue;
     std::sort(per[p].begin(), per[p].end());
     pt2t[p] = NT++;
     for (auto& e : per[p]) {
+      if ((int)tj.size() == tjstart.back() || tj.back() != e.first) tj.push_back(e.first);
       ejp.push_back(e.first);
       elma.push_back(e.second);
     }
     tstart.push_back((int)ejp.size());
+    tjstart.push_back((int)tj.size());
   }
   // the old tables, projection and work buffers go: drop graphs that captured them
   (void)hipStreamSynchronize(c->stream);
@@ -1068,7 +1070,9 @@ int salmon_gpu_set_projectors(salmon_ctx* c, int NI, int Nps, const int* Mps, co
       (r = up(pt2t.data(), sizeof(int) * pt2t.size(), (void**)&kb.pt2t)) ||
       (r = up(tstart.data(), sizeof(int) * tstart.size(), (void**)&kb.t_start)) ||
       (r = up(elma.data(), sizeof(int) * elma.size(), (void**)&kb.e_lma)) ||
-      (r = up(ejp.data(), sizeof(int) * ejp.size(), (void**)&kb.e_jp)))
+      (r = up(ejp.data(), sizeof(int) * ejp.size(), (void**)&kb.e_jp)) ||
+      (r = up(tjstart.data(), sizeof(int) * tjstart.size(), (void**)&kb.tj_start)) ||
+      (r = up(tj.data(), sizeof(int) * tj.size(), (void**)&kb.tj)))
     return r;
   c->kb = kb;
   c->kb_host = {start, pidx, atom_lma, pos, std::vector<double>(uV, uV + (size_t)Nps * Nlma), sign};

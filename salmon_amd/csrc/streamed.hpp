@@ -219,11 +219,10 @@ __global__ void __launch_bounds__(256) k_phase_table(const double* __restrict__ 
 // with A = (|k|^2 - sum lap0)/2, C = lap/H^2, D = k.nab/H.
 // tt (nullable) gets F - V E before the KB term (hpsi.f90:131-133).
 // ---------------------------------------------------------------------------
+// the terms before KB; e = E(p) and V = vloc(p)
 template <typename T>
-__device__ __forceinline__ cplx<T> hpsi_point(const cplx<T>* __restrict__ E, int p, double kx, double ky, double kz,
-                                              const T* __restrict__ vloc, const Grid& g, const KBTables& kb,
-                                              const cplx<T>* __restrict__ U, cplx<T>* __restrict__ ttp,
-                                              const cplx<T>* __restrict__ ph = nullptr) {
+__device__ __forceinline__ cplx<T> stencil_point(const cplx<T>* __restrict__ E, int p, double kx, double ky, double kz,
+                                                 const T* __restrict__ vloc, const Grid& g, cplx<T>& e, T& V) {
   const T A = (T)((kx * kx + ky * ky + kz * kz - (g.lap[0][0] + g.lap[1][0] + g.lap[2][0])) * 0.5);
   const int NLx = g.NLx, NLy = g.NLy, NLz = g.NLz;
   const int iz = p % NLz, iy = (p / NLz) % NLy, ix = p / (NLz * NLy);
@@ -250,11 +249,22 @@ __device__ __forceinline__ cplx<T> hpsi_point(const cplx<T>* __restrict__ E, int
       wi += D * (ep.im - em.im);
     }
   }
-  const cplx<T> e = E[p];
-  const T V = vloc[p];
+  e = E[p];
+  V = vloc[p];
   cplx<T> f;
   f.re = (V + A) * e.re - (T)0.5 * vr + wi;
   f.im = (V + A) * e.im - (T)0.5 * vi - wr;
+  return f;
+}
+
+template <typename T>
+__device__ __forceinline__ cplx<T> hpsi_point(const cplx<T>* __restrict__ E, int p, double kx, double ky, double kz,
+                                              const T* __restrict__ vloc, const Grid& g, const KBTables& kb,
+                                              const cplx<T>* __restrict__ U, cplx<T>* __restrict__ ttp,
+                                              const cplx<T>* __restrict__ ph = nullptr) {
+  cplx<T> e;
+  T V;
+  cplx<T> f = stencil_point<T>(E, p, kx, ky, kz, vloc, g, e, V);
   if (ttp) *ttp = cplx<T>{f.re - V * e.re, f.im - V * e.im};
   const int t = kb.pt2t[p];
   if (t >= 0) {
