@@ -20,7 +20,11 @@ namespace cg {
 constexpr int kPPT = 2;              // points per thread of a projection block
 constexpr int kChunk = 256 * kPPT;   // points per projection block
 constexpr int kJG = 8;               // lower bands per projection block
-constexpr int kSubPts = 64;          // points per subtraction block, one per lane; its waves share the bands
+// The subtractions run in blocks of 1024 threads: every block of a k point arrives
+// at one counter, and those atomics are served one by one (per launch, 32^3 and 8 k
+// points of 16^3: 9.4 and 10.7 us with blocks of 64 points, 8.2 and 8.7 of 256).
+constexpr int kWide = 1024;
+constexpr int kSubPts = 256;  // points per subtraction block; its waves share the bands
 
 // per-k scalars (double slots)
 enum : int {
@@ -52,11 +56,28 @@ constexpr int kPartQ = 2 * kJG;
 // order.  Returns true in the block that arrives last; there, tot[] holds the
 // totals in thread 0.  Its threads load the partials side by side: one thread
 // reading them in block order took 1 to 3 us per launch on 32 to 128 blocks.
-template <int NQ>
+template <int NQ, int NT = 256>
 __device__ bool last_block_sum(double (&v)[NQ], const State& S, int nblk, int bid, double (&tot)[NQ]) {
-  __shared__ double smem[4 * NQ];
+  constexpr int NW = NT / kWave;
+  __shared__ double smem[NW * NQ];
   __shared__ int is_last;
-  block_sum256<NQ>(v, smem);
+  const int lane = threadIdx.x & (kWave - 1), wv = threadIdx.x / kWave;
+  auto block = [&](double (&a)[NQ]) {  // valid in thread 0
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) a[q] = wave_sum(a[q]);
+    if (lane == 0) {
+#pragma unroll
+      for (int q = 0; q < NQ; ++q) smem[wv * NQ + q] = a[q];
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+#pragma unroll
+      for (int q = 0; q < NQ; ++q)
+        for (int w = 1; w < NW; ++w) a[q] += smem[w * NQ + q];
+    }
+    __syncthreads();
+  };
+  block(v);
   const int k = blockIdx.y;
   double* part = S.part + (size_t)k * S.pstride;
   if (threadIdx.x == 0) {
@@ -71,11 +92,11 @@ __device__ bool last_block_sum(double (&v)[NQ], const State& S, int nblk, int bi
   if (!is_last) return false;
 #pragma unroll
   for (int q = 0; q < NQ; ++q) tot[q] = 0.0;
-  for (int b = threadIdx.x; b < nblk; b += 256) {
+  for (int b = threadIdx.x; b < nblk; b += NT) {
 #pragma unroll
     for (int q = 0; q < NQ; ++q) tot[q] += __hip_atomic_load(&part[b * NQ + q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
-  block_sum256<NQ>(tot, smem);
+  block(tot);
   return true;
 }
 
@@ -128,7 +149,7 @@ __global__ void __launch_bounds__(256) k_cg_proj(State S, const cplx<double>* __
                                                  int mode, int check_done) {
   const int k = blockIdx.z;
   const int skip = check_done ? S.done[k] : 0;
-  const int c = blockIdx.x, g0 = blockIdx.y * kJG;
+  const int t = threadIdx.x, c = blockIdx.x, g0 = blockIdx.y * kJG;
   const int nj = min(kJG, ib - g0);
   const double xhx = S.sc[k * kNS + XHX];
   const cplx<double>* B = zu + (size_t)k * S.NB * S.NL;
@@ -144,7 +165,7 @@ __global__ void __launch_bounds__(256) k_cg_proj(State S, const cplx<double>* __
   bool okp[kPPT];
 #pragma unroll
   for (int i = 0; i < kPPT; ++i) {
-    const int p = c * kChunk + i * 256 + threadIdx.x;
+    const int p = c * kChunk + i * 256 + t;
     okp[i] = p < S.NL;
     pc[i] = okp[i] ? p : 0;
   }
@@ -158,7 +179,7 @@ __global__ void __launch_bounds__(256) k_cg_proj(State S, const cplx<double>* __
   }
 #pragma unroll
   for (int j = 0; j < kJG; ++j) {
-    const int jb = g0 + (j < nj ? j : nj - 1);
+    const int jb = min(g0 + j, ib - 1);
 #pragma unroll
     for (int i = 0; i < kPPT; ++i) {
       const cplx<double> b0 = B[(size_t)jb * S.NL + pc[i]];
@@ -170,73 +191,82 @@ __global__ void __launch_bounds__(256) k_cg_proj(State S, const cplx<double>* __
   }
   loaded(cplx<double>{acc[0], acc[2 * kJG - 1]});
   if (skip) return;
-  // partials: [group][chunk][2*kJG]
-  __shared__ double smem[4 * kPartQ];
+  // partials: [chunk][group][2*kJG]
+  __shared__ double smem[256];
   __shared__ int is_last;
-  const int t = threadIdx.x, lane = t & (kWave - 1), wv = t / kWave;
+  const int lane = t & (kWave - 1), wv = t / kWave, np = gridDim.y * kPartQ;
   wave_sums(acc);
 #pragma unroll
   for (int q = 0; q < kPartQ; ++q)
     if (lane == wave_sums_lane(q)) smem[wv * kPartQ + q] = acc[0];
   double* part = S.part + (size_t)k * S.pstride;
-  const int nblk = S.nchunk * gridDim.y;
-  const int bid = blockIdx.y * S.nchunk + c;
   __syncthreads();
-  if (wv == 0) {  // one wave stores them and arrives: its stores are ordered before its arrival
-    if (lane < kPartQ) {
-      const double v = (smem[lane] + smem[kPartQ + lane]) + (smem[2 * kPartQ + lane] + smem[3 * kPartQ + lane]);
-      __hip_atomic_store(&part[(size_t)bid * kPartQ + lane], v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
+  if (t < kPartQ) {
+    const double v = (smem[t] + smem[kPartQ + t]) + (smem[2 * kPartQ + t] + smem[3 * kPartQ + t]);
+    __hip_atomic_store(&part[(size_t)c * np + blockIdx.y * kPartQ + t], v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     agent_stores_done();
-    if (lane == 0) {
-      const unsigned n = agent_arrive(&S.cnt[k]);
-      is_last = (n == (unsigned)(nblk - 1));
-      if (is_last) __hip_atomic_store(&S.cnt[k], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
+  }
+  if (t == 0) {  // (in the wave that stored)
+    is_last = agent_arrive(&S.cnt[k]) == gridDim.x * gridDim.y - 1;
+    if (is_last) __hip_atomic_store(&S.cnt[k], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
   __syncthreads();
   if (!is_last) return;
-  // The last block of row k: four threads per band (quad qd, part qi), each
-  // taking every fourth term of a sum with kTailBatch loads in flight (clamped
-  // indices, terms past the end zero), then the quad's sum in a fixed order.
-  // One thread per band left this to 64 lanes and up to 64 dependent loads.
-  __shared__ cplx<double> zsh[kCgMaxNB];
-  constexpr int kTailBatch = 16;
-  const int qd = t >> 2, qi = t & 3;
-  auto quad = [](double v) {
-    v += dpp_mov<dpp::kQuad1032, 0xf>(v);
-    return v + dpp_mov<dpp::kQuad2301, 0xf>(v);
-  };
-  for (int j0 = 0; j0 < ib; j0 += 64) {
-    const int j = j0 + qd, jc = min(j, ib - 1), grp = jc / kJG, jj = jc % kJG;
-    double sr = 0.0, si = 0.0;
-    for (int c0 = qi; c0 < S.nchunk; c0 += 4 * kTailBatch) {
-      double vr[kTailBatch], vi[kTailBatch];
-#pragma unroll
-      for (int u = 0; u < kTailBatch; ++u) {
-        const size_t b = (size_t)(grp * S.nchunk + min(c0 + 4 * u, S.nchunk - 1)) * kPartQ;
-        vr[u] = __hip_atomic_load(&part[b + 2 * jj], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        vi[u] = __hip_atomic_load(&part[b + 2 * jj + 1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      }
-#pragma unroll
-      for (int u = 0; u < kTailBatch; ++u) {
-        const bool ok = c0 + 4 * u < S.nchunk;
-        sr = ok ? sr + vr[u] : sr;
-        si = ok ? si + vi[u] : si;
-      }
-    }
-    sr = quad(sr);
-    si = quad(si);
-    if (qi == 0 && j < ib) zsh[j] = cplx<double>{sr * S.Hxyz, si * S.Hxyz};
-  }
-  __syncthreads();
+  // The last block of row k, which the launch waits for: its loads are few rounds
+  // of many in flight.  The first of the inverse's rows, which do not depend on the
+  // sums, come with them: four threads (quad qd, part qi) per row, each every
+  // fourth column.
   cplx<double>* gram = S.gram + (size_t)k * S.NB * S.NB;
   cplx<double>* M = S.minv + (size_t)k * S.NB * S.NB;
   double* MR = S.minvr + (size_t)k * S.NB * S.NB;
+  constexpr int kTail = 16;
+  const int qd = t >> 2, qi = t & 3;
+  cplx<double> mm[kTail];
+  auto row = [&](int j0, int l0) {  // M(j0 + qd, l0 + qi + 4 u), l < j; clamped elsewhere
+    const int j = min(j0 + qd, ib - 1);
+#pragma unroll
+    for (int u = 0; u < kTail; ++u) {
+      const size_t o = (size_t)j * S.NB + min(l0 + qi + 4 * u, j);
+      if (mode == PROJ_START) mm[u] = cplx<double>{MR[o], 0.0};
+      else mm[u] = M[o];
+    }
+  };
+  if (mode == PROJ_START || mode == PROJ_VEC) row(0, 0);
+  // sums over the chunks: thread (value, share of the chunks), then the shares in order
+  __shared__ cplx<double> zsh[kCgMaxNB];
+  double* zv = (double*)zsh;
+  int lg = 0;
+  while ((1 << lg) < 2 * ib && lg < 8) ++lg;
+  const int nv = 1 << lg, ns = 256 >> lg, sh = t >> lg;
+  for (int v0 = 0; v0 < 2 * ib; v0 += nv) {
+    const int v = v0 + (t & (nv - 1)), vc = min(v, 2 * ib - 1);
+    double s = 0.0;
+    for (int c0 = sh; c0 < S.nchunk; c0 += 8 * ns) {
+      double a[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        a[u] = __hip_atomic_load(&part[(size_t)min(c0 + u * ns, S.nchunk - 1) * np + vc], __ATOMIC_RELAXED,
+                                 __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+      for (int u = 0; u < 8; ++u) s = c0 + u * ns < S.nchunk ? s + a[u] : s;
+    }
+    __syncthreads();
+    smem[t] = s;
+    __syncthreads();
+    if (sh == 0 && v < 2 * ib) {
+      for (int r = 1; r < ns; ++r) s += smem[r * nv + t];
+      zv[v] = s * S.Hxyz;
+    }
+  }
+  __syncthreads();
   if (mode == PROJ_PLAIN) {  // coefficients against the unmodified vector
     for (int j = t; j < ib; j += 256) S.zs[(size_t)k * S.NB + j] = zsh[j];
     return;
   }
+  auto quad = [](double v) {
+    v += dpp_mov<dpp::kQuad1032, 0xf>(v);
+    return v + dpp_mov<dpp::kQuad2301, 0xf>(v);
+  };
   if (mode == PROJ_GRAM) {
     // raw_j = Hxyz <B_j|B_ib>, so G(ib, j) = conj(raw_j)
     for (int j = t; j < ib; j += 256) gram[(size_t)ib * S.NB + j] = cplx<double>{zsh[j].re, -zsh[j].im};
@@ -248,17 +278,16 @@ __global__ void __launch_bounds__(256) k_cg_proj(State S, const cplx<double>* __
         sr = rr = zsh[lc].re;
         si = -zsh[lc].im;
       }
-      for (int q0 = j0 + qi; q0 < ib; q0 += 4 * kTailBatch) {
-        cplx<double> mm[kTailBatch];
-        double mr[kTailBatch];
+      for (int q0 = j0 + qi; q0 < ib; q0 += 4 * kTail) {
+        double mr[kTail];
 #pragma unroll
-        for (int u = 0; u < kTailBatch; ++u) {
+        for (int u = 0; u < kTail; ++u) {
           const size_t o = (size_t)max(min(q0 + 4 * u, ib - 1), lc) * S.NB + lc;  // (row q > column l, or not used)
           mm[u] = M[o];
           mr[u] = MR[o];
         }
 #pragma unroll
-        for (int u = 0; u < kTailBatch; ++u) {
+        for (int u = 0; u < kTail; ++u) {
           const int q = q0 + 4 * u;
           const bool ok = q > l && q < ib;
           const cplx<double> z = zsh[min(q, ib - 1)];
@@ -277,41 +306,25 @@ __global__ void __launch_bounds__(256) k_cg_proj(State S, const cplx<double>* __
     }
     return;
   }
-  // c = M b
+  // c = M b (PROJ_START: of the real parts)
+  const bool real = mode == PROJ_START;
   for (int j0 = 0; j0 < ib; j0 += 64) {
-    const int j = j0 + qd, jc = min(j, ib - 1);
-    double cr = 0.0, ci = 0.0;
-    if (qi == 0) {
-      cr = zsh[jc].re;
-      ci = mode == PROJ_START ? 0.0 : zsh[jc].im;
-    }
-    const int l1 = min(ib, j0 + 64);  // columns below the rows of this pass
-    for (int l0 = qi; l0 < l1; l0 += 4 * kTailBatch) {
-      if (mode == PROJ_START) {
-        double mr[kTailBatch];
+    const int j = min(j0 + qd, ib - 1);
+    double cr = qi == 0 ? zsh[j].re : 0.0, ci = qi == 0 && !real ? zsh[j].im : 0.0;
+    for (int l0 = 0; l0 < min(ib, j0 + 64); l0 += 4 * kTail) {
+      if (j0 > 0 || l0 > 0) row(j0, l0);
 #pragma unroll
-        for (int u = 0; u < kTailBatch; ++u) mr[u] = MR[(size_t)jc * S.NB + min(l0 + 4 * u, jc)];
-#pragma unroll
-        for (int u = 0; u < kTailBatch; ++u) {
-          const int l = l0 + 4 * u;
-          cr = l < jc ? cr + mr[u] * zsh[min(l, jc)].re : cr;
-        }
-      } else {
-        cplx<double> mm[kTailBatch];
-#pragma unroll
-        for (int u = 0; u < kTailBatch; ++u) mm[u] = M[(size_t)jc * S.NB + min(l0 + 4 * u, jc)];
-#pragma unroll
-        for (int u = 0; u < kTailBatch; ++u) {
-          const int l = l0 + 4 * u;
-          const cplx<double> m = mm[u], z = zsh[min(l, jc)];
-          cr = l < jc ? cr + (m.re * z.re - m.im * z.im) : cr;
-          ci = l < jc ? ci + (m.re * z.im + m.im * z.re) : ci;
-        }
+      for (int u = 0; u < kTail; ++u) {
+        const int l = l0 + qi + 4 * u;
+        const cplx<double> m = mm[u], z = zsh[min(l, j)];
+        const double zi = real ? 0.0 : z.im;
+        cr = l < j ? cr + (m.re * z.re - m.im * zi) : cr;
+        ci = l < j ? ci + (m.re * zi + m.im * z.re) : ci;
       }
     }
     cr = quad(cr);
     ci = quad(ci);
-    if (qi == 0 && j < ib) S.zs[(size_t)k * S.NB + j] = cplx<double>{cr, ci};
+    if (qi == 0 && j0 + qd < ib) S.zs[(size_t)k * S.NB + j] = cplx<double>{cr, ci};
   }
 }
 
@@ -331,46 +344,48 @@ enum : int {
 // finisher forms the conjugation ratio uk = s/gkgk (CG.f90:92-98; iteration 1
 // takes p = d) and, from <x|d> and <x|p_old>, the overlap zs = <x|d + uk p_old>
 // that the direction is stripped of (CG.f90:103), so p needs no pass of its own.
-// A block's lanes are its points and its four waves take every fourth band: the
-// loop's loads are the launch's time (64 bands of 32^3: 8 loads in flight per
-// lane, two rounds of them instead of eight).  Grid (nsub, NK).
-__global__ void __launch_bounds__(256) k_cg_sub(State S, const cplx<double>* __restrict__ zu, int ib, Src src,
+// Each quarter of a block takes every fourth band for the block's points, whose
+// sum the first quarter forms: the loop's loads are the launch's time (64 bands:
+// 8 loads in flight per lane, two rounds of them instead of eight).
+// Grid (nsub, NK), kWide threads.
+__global__ void __launch_bounds__(kWide) k_cg_sub(State S, const cplx<double>* __restrict__ zu, int ib, Src src,
                                                 cplx<double>* out, const cplx<double>* __restrict__ other,
                                                 const cplx<double>* __restrict__ x, const cplx<double>* __restrict__ P,
                                                 int role, int it, int ncg) {
   const int k = blockIdx.y;
   const int skip = role != SUB_START ? S.done[k] : 0;
-  const int c = blockIdx.x, lane = threadIdx.x & (kWave - 1), wv = threadIdx.x / kWave;
+  const int c = blockIdx.x, t = threadIdx.x & (kSubPts - 1);
+  const int part = __builtin_amdgcn_readfirstlane(threadIdx.x / kSubPts);
   const size_t off = (size_t)k * S.NL;
   const double xhx = S.sc[k * kNS + XHX];
   const cplx<double>* B = zu + (size_t)k * S.NB * S.NL;
   const cplx<double>* zs = S.zs + (size_t)k * S.NB;
-  const int p = c * kSubPts + lane, pc = min(p, S.NL - 1);
+  const int p = c * kSubPts + t, pc = min(p, S.NL - 1);
   const bool dir = role != SUB_START && role != SUB_NONE;
   cplx<double> e{0, 0}, o{0, 0}, xp{0, 0}, q{0, 0};
-  if (wv == 0) {
+  if (part == 0) {
     e = src.at(k, S.NL, pc, xhx);
     if (role == SUB_PCDIR) o = other[off + pc];
     if (dir) xp = x[off + pc];
     if (dir && it > 1 && role != SUB_LEARN) q = P[off + pc];
   }
 #pragma unroll 8
-  for (int j = wv; j < ib; j += 4) {
+  for (int j = part; j < ib; j += 4) {
     const cplx<double> b = B[(size_t)j * S.NL + pc], z = zs[j];
     e.re -= b.re * z.re - b.im * z.im;
     e.im -= b.re * z.im + b.im * z.re;
   }
   loaded(e);
   if (skip) return;
-  __shared__ cplx<double> sh[3][kWave];
-  if (wv > 0) sh[wv - 1][lane] = e;
+  __shared__ cplx<double> sh[3][kSubPts];
+  if (part > 0) sh[part - 1][t] = e;
   __syncthreads();
   double v[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-  if (wv == 0 && p < S.NL) {
+  if (part == 0 && p < S.NL) {
 #pragma unroll
     for (int w = 0; w < 3; ++w) {
-      e.re += sh[w][lane].re;
-      e.im += sh[w][lane].im;
+      e.re += sh[w][t].re;
+      e.im += sh[w][t].im;
     }
     out[off + p] = e;
     v[0] = role == SUB_PCDIR ? e.re * o.re + e.im * o.im : e.re * e.re + e.im * e.im;
@@ -381,7 +396,7 @@ __global__ void __launch_bounds__(256) k_cg_sub(State S, const cplx<double>* __r
   }
   if (role == SUB_NONE) return;
   double tot[5];
-  if (!last_block_sum<5>(v, S, S.nsub, c, tot)) return;
+  if (!last_block_sum<5, kWide>(v, S, S.nsub, c, tot)) return;
   if (threadIdx.x != 0) return;
   double* sc = S.sc + k * kNS;
   if (role == SUB_START) {

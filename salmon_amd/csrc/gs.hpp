@@ -273,7 +273,7 @@ static int cg_run(salmon_ctx* c, int ncg, int precond) {
     return SALMON_OK;
   };
   auto sub = [&](int ib, Src src, cplx<double>* out, const cplx<double>* other, int role, int it) -> int {
-    hipLaunchKernelGGL(k_cg_sub, gsub, blk, 0, c->stream, S, (const cplx<double>*)zu, ib, src, out, other,
+    hipLaunchKernelGGL(k_cg_sub, gsub, dim3(kWide), 0, c->stream, S, (const cplx<double>*)zu, ib, src, out, other,
                        (const cplx<double>*)w[W_X], (const cplx<double>*)w[W_P], role, it, ncg);
     LAUNCHCHK(c);
     return SALMON_OK;
