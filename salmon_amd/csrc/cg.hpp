@@ -12,6 +12,7 @@
 // A k whose band met the exit test (|ev - <x|H|x>| < 1e-15, CG.f90:114)
 // skips the remaining iteration kernels.
 #pragma once
+#include "dft.hpp"
 #include "streamed.hpp"
 
 namespace salmon {
@@ -691,95 +692,47 @@ __global__ void __launch_bounds__(256) k_cg_resid(State S, const cplx<double>* _
 // Kinetic preconditioner K g = F^-1 [ k(x) F g ], x = t(q)/<x|T|x>, with t(q)
 // the finite-difference kinetic symbol -1/2 sum_axes (lap0 + 2 sum_m lap_m
 // cos(m q h)) and k(x) = f/(f + 16 x^4), f = 27 + 18x + 12x^2 + 8x^3 (the
-// Teter-Payne-Allan form).  The 3-D transform is three passes of 1-D DFTs
-// along z, y and x (direct sums over a line held in LDS, twiddles from a
-// table, line length <= kDftMax); the x pass applies k(x) between its forward
-// and inverse transforms.  No reference counterpart: CG_ompk applies no
-// preconditioner (CG.f90:85-92).
+// Teter-Payne-Allan form), in the three launches of dft.hpp (a pass per axis, five
+// launches, took 30 us on 32^3).  No reference counterpart: CG_ompk applies no
+// preconditioner (CG.f90:85-92).  Twiddles (cos, sin)(2 pi j/n) of axis a at
+// tw + 2 * kDftMax * a, symbols at symb + kDftMax * a.
 // ---------------------------------------------------------------------------
 constexpr int kDftMax = 64;
 
-struct DftAxis {
-  int n;       // line length
-  int es;      // element stride
-  int nlines;  // lines of the axis
-  int lpb;     // lines per block
-};
-
-// line l of axis a -> base offset (z: l*NLz; y: ix*NLy*NLz + iz with l = ix*NLz + iz;
-// x: l with l = iy*NLz + iz)
-__device__ __forceinline__ int dft_line_base(int axis, int l, const Grid& g) {
-  if (axis == 2) return l * g.NLz;
-  if (axis == 1) return (l / g.NLz) * g.NLy * g.NLz + (l % g.NLz);
-  return l;
+// Grid (blocks of z lines, NLx, NK).
+__global__ void __launch_bounds__(256) k_kin_zy(State S, const cplx<double>* __restrict__ in, cplx<double>* __restrict__ out,
+                                                Grid g, const double* __restrict__ tw) {
+  const int k = blockIdx.z;
+  if (S.done[k]) return;
+  const size_t o = (size_t)k * g.NL + (size_t)blockIdx.y * g.NLy * g.NLz;
+  dft::plane<true>(g.NLz, g.NLy, tw + 4 * kDftMax, tw + 2 * kDftMax, -1.0,
+                   [&](int z, int y) { return in[o + y * g.NLz + z]; },
+                   [&](int z, int y, cplx<double> v) { out[o + y * g.NLz + z] = v; });
 }
 
-// One DFT pass.  dir = -1 forward (exp(-2 pi i c m/n)), +1 inverse (scaled by
-// 1/n).  For axis x with symb != nullptr: forward, times k(x), inverse.
-// tw = (cos, sin)(2 pi j/n), j = 0..n-1, per axis at tw + axis*kDftMax.
-__global__ void __launch_bounds__(256) k_dft_pass(const State S, const cplx<double>* __restrict__ in,
-                                                  cplx<double>* __restrict__ out, Grid g, int axis, int dir,
-                                                  const double* __restrict__ tw, const double* __restrict__ symb,
-                                                  int check_done) {
+// Grid (blocks of x lines, NK).
+__global__ void __launch_bounds__(256) k_kin_x(State S, cplx<double>* __restrict__ f, Grid g, const double* __restrict__ tw,
+                                               const double* __restrict__ symb) {
   const int k = blockIdx.y;
-  if (check_done && S.done[k]) return;
-  const int n = axis == 2 ? g.NLz : (axis == 1 ? g.NLy : g.NLx);
-  const int es = axis == 2 ? 1 : (axis == 1 ? g.NLz : g.NLy * g.NLz);
-  const int nlines = g.NL / n;
-  const int lpb = 256 / n;
-  const int l0 = blockIdx.x * lpb;
-  __shared__ cplx<double> s[256 + 8];
-  __shared__ double2 w[kDftMax];
-  for (int j = threadIdx.x; j < n; j += 256) w[j] = make_double2(tw[2 * (axis * kDftMax + j)], tw[2 * (axis * kDftMax + j) + 1]);
-  const size_t off = (size_t)k * g.NL;
-  // element e of line l sits at s[li*n + e]; z lines load contiguously,
-  // y and x lines with consecutive lines on consecutive threads
-  const int t = threadIdx.x;
-  int li, e;
-  if (axis == 2) { li = t / n; e = t % n; } else { li = t % lpb; e = t / lpb; }
-  const bool active = t < lpb * n && (l0 + li) < nlines;
-  const int base = active ? dft_line_base(axis, l0 + li, g) : 0;
-  if (active) s[li * n + e] = in[off + base + (size_t)e * es];
-  __syncthreads();
-  auto dft = [&](int sgn) -> cplx<double> {
-    double re = 0.0, im = 0.0;
-    const cplx<double>* a = s + li * n;
-    int j = 0;
-    for (int m = 0; m < n; ++m) {
-      const double c = w[j].x, sn = sgn * w[j].y;
-      re += c * a[m].re - sn * a[m].im;
-      im += c * a[m].im + sn * a[m].re;
-      j += e;
-      if (j >= n) j -= n;
-    }
-    return cplx<double>{re, im};
-  };
-  cplx<double> r{0.0, 0.0};
-  if (active) r = dft(dir);
-  if (symb) {
-    // x pass: forward done; multiply by k(x) and transform back
-    __syncthreads();
-    if (active) {
-      const int l = l0 + li, iy = l / g.NLz, iz = l % g.NLz;
-      const double tq = (symb[e] + symb[kDftMax + iy]) + symb[2 * kDftMax + iz];
-      double txx = S.sc[k * kNS + XTX];
-      if (!(txx > 1e-12)) txx = 1e-12;
-      const double x = tq / txx;
-      const double f = 27.0 + 18.0 * x + 12.0 * x * x + 8.0 * x * x * x;
-      const double kf = f / (f + 16.0 * x * x * x * x);
-      s[li * n + e] = cplx<double>{kf * r.re, kf * r.im};
-    }
-    __syncthreads();
-    if (active) r = dft(+1);
-  }
-  if (active) {
-    if (dir > 0 || symb) {
-      const double inv = 1.0 / n;
-      r.re *= inv;
-      r.im *= inv;
-    }
-    out[off + base + (size_t)e * es] = r;
-  }
+  if (S.done[k]) return;
+  double txx = S.sc[k * kNS + XTX];
+  if (!(txx > 1e-12)) txx = 1e-12;
+  dft::lines_x(g, f + (size_t)k * g.NL, tw, [&](int ix, int iy, int iz) {
+    const double x = ((symb[ix] + symb[kDftMax + iy]) + symb[2 * kDftMax + iz]) / txx;
+    const double q = 27.0 + 18.0 * x + 12.0 * x * x + 8.0 * x * x * x;
+    return q / (q + 16.0 * x * x * x * x) / g.NL;
+  });
+}
+
+// Grid (blocks of y lines, NLx, NK).
+__global__ void __launch_bounds__(256) k_kin_yz(State S, const cplx<double>* __restrict__ in, cplx<double>* __restrict__ out,
+                                                Grid g, const double* __restrict__ tw) {
+  const int k = blockIdx.z;
+  if (S.done[k]) return;
+  const size_t o = (size_t)k * g.NL + (size_t)blockIdx.y * g.NLy * g.NLz;
+  dft::plane<false>(g.NLy, g.NLz, tw + 2 * kDftMax, tw + 4 * kDftMax, 1.0,
+                    [&](int y, int z) { return in[o + y * g.NLz + z]; },
+                    [&](int y, int z, cplx<double> v) { out[o + y * g.NLz + z] = v; });
 }
 
 // ---------------------------------------------------------------------------

@@ -21,7 +21,7 @@ struct PcInfer {
 struct GsState {
   int NK = 0, NB = 0, NL = 0, Nlma = 0, NPI = 0, nchunk = 0, ngroup = 0;
   std::vector<void*> bufs;
-  cplx<double>* w[11] = {};  // X HX TX G P PKO HP TP KG T1 T2, NK*NL each
+  cplx<double>* w[10] = {};  // X HX TX G P PKO HP TP KG T1, NK*NL each
   cplx<double>* ph = nullptr;   // (NK, NPI) phases of the sphere points at the CG's k
   cplx<double>* dps = nullptr;  // (NK, NPI) KB term of each
   double* sc = nullptr;
@@ -79,7 +79,7 @@ static void graph_free(GsState::Graph& g) {
 
 static int pc_infer(salmon_ctx* c, GsState* s, salmon_pcnet* net, const cplx<double>* g, cplx<double>* out);
 
-enum { W_X = 0, W_HX, W_TX, W_G, W_P, W_PKO, W_HP, W_TP, W_KG, W_T1, W_T2 };
+enum { W_X = 0, W_HX, W_TX, W_G, W_P, W_PKO, W_HP, W_TP, W_KG, W_T1 };
 
 static void gs_free(salmon_ctx* c) {
   GsState* s = (GsState*)c->gs;
@@ -137,7 +137,7 @@ static int gs_ensure(salmon_ctx* c) {
   s->pstride = std::max(s->nchunk * s->ngroup * kPartQ, (s->NL + kSubPts - 1) / kSubPts * 5);
   const size_t nv = (size_t)s->NK * s->NL;
   int r;
-  for (int i = 0; i < 11; ++i)
+  for (int i = 0; i < 10; ++i)
     if ((r = gs_alloc(c, s, &s->w[i], nv))) return r;
   if ((r = gs_alloc(c, s, &s->ph, (size_t)s->NK * s->NPI))) return r;
   if ((r = gs_alloc(c, s, &s->dps, (size_t)s->NK * s->NPI))) return r;
@@ -206,26 +206,19 @@ static State gs_view(salmon_ctx* c, GsState* s) {
   return S;
 }
 
-// K g for the kinetic preconditioner: five DFT passes g -> T1 -> T2 -> T1 -> T2 -> out.
+// K g for the kinetic preconditioner.
 static int kinetic_apply(salmon_ctx* c, GsState* s, const State& S, const cplx<double>* g, cplx<double>* out) {
+  namespace dft = salmon::dft;
   const Grid& G = c->g;
-  cplx<double>* t1 = s->w[W_T1];
-  cplx<double>* t2 = s->w[W_T2];
-  auto pass = [&](const cplx<double>* in, cplx<double>* o, int axis, int dir, const double* symb) -> int {
-    const int n = axis == 2 ? G.NLz : (axis == 1 ? G.NLy : G.NLx);
-    const int lpb = 256 / n;
-    const int nl = G.NL / n;
-    hipLaunchKernelGGL(k_dft_pass, dim3((nl + lpb - 1) / lpb, s->NK), dim3(256), 0, c->stream, S, in, o, G, axis, dir,
-                       s->tw, symb, 1);
-    LAUNCHCHK(c);
-    return SALMON_OK;
-  };
-  int r;
-  if ((r = pass(g, t1, 2, -1, nullptr))) return r;
-  if ((r = pass(t1, t2, 1, -1, nullptr))) return r;
-  if ((r = pass(t2, t1, 0, -1, s->symb))) return r;
-  if ((r = pass(t1, t2, 1, +1, nullptr))) return r;
-  return pass(t2, out, 2, +1, nullptr);
+  const int nz = dft::plane_lines(G.NLy), ny = dft::plane_lines(G.NLz);
+  hipLaunchKernelGGL(k_kin_zy, dim3((G.NLz + nz - 1) / nz, G.NLx, s->NK), dim3(256), dft::plane_lds(G.NLz, G.NLy), c->stream, S,
+                     g, s->w[W_T1], G, (const double*)s->tw);
+  hipLaunchKernelGGL(k_kin_x, dim3(dft::lines_x_blocks(G), s->NK), dim3(256), 0, c->stream, S, s->w[W_T1], G,
+                     (const double*)s->tw, (const double*)s->symb);
+  hipLaunchKernelGGL(k_kin_yz, dim3((G.NLy + ny - 1) / ny, G.NLx, s->NK), dim3(256), dft::plane_lds(G.NLy, G.NLz), c->stream, S,
+                     (const cplx<double>*)s->w[W_T1], out, G, (const double*)s->tw);
+  LAUNCHCHK(c);
+  return SALMON_OK;
 }
 
 // CG_ompk over all bands of all k (FP64 orbitals).  An iteration is a chain of

@@ -500,31 +500,22 @@ void scf_twiddles(const Grid& g, double* tw) {
 }
 
 // V_H and V_xc of the device density rho with the twiddles tw and two complex
-// grids A, B (device): Hartree by per-axis DFTs and the Coulomb kernel, then
+// grids A, B (device): Hartree by DFTs and the Coulomb kernel, then
 // Vloc = V_H + Vpsl + V_xc into the context's potential (set_v) and/or the
 // parts into vh, vxc (device, nullable).  Launches only.
 int scf_potential_on(salmon_ctx* c, const double* rho, bool set_v, int xc, double* vh, double* vxc, const double* tw,
                      cplx<double>* A, cplx<double>* B) {
+  namespace dft = salmon::dft;
   const Grid& g = c->g;
-  const dim3 gr((g.NL + 255) / 256), bl(256);
-  hipLaunchKernelGGL(salmon::scf::k_real_to_cplx, gr, bl, 0, c->stream, rho, A, g.NL);
-  hipLaunchKernelGGL(salmon::scf::k_dft_axis, gr, bl, 0, c->stream, (const cplx<double>*)A, B, g, 2, -1, tw);
-  hipLaunchKernelGGL(salmon::scf::k_dft_axis, gr, bl, 0, c->stream, (const cplx<double>*)B, A, g, 1, -1, tw);
-  hipLaunchKernelGGL(salmon::scf::k_dft_axis, gr, bl, 0, c->stream, (const cplx<double>*)A, B, g, 0, -1, tw);
-  hipLaunchKernelGGL(salmon::scf::k_coulomb, gr, bl, 0, c->stream, B, g);
-  hipLaunchKernelGGL(salmon::scf::k_dft_axis, gr, bl, 0, c->stream, (const cplx<double>*)B, A, g, 2, +1, tw);
-  hipLaunchKernelGGL(salmon::scf::k_dft_axis, gr, bl, 0, c->stream, (const cplx<double>*)A, B, g, 1, +1, tw);
-  hipLaunchKernelGGL(salmon::scf::k_dft_axis, gr, bl, 0, c->stream, (const cplx<double>*)B, A, g, 0, +1, tw);
-  LAUNCHCHK(c);
-  if (set_v) {
-    hipLaunchKernelGGL(salmon::scf::k_vloc, gr, bl, 0, c->stream, (const cplx<double>*)A, rho, (const double*)c->d_vpsl,
-                       xc, g.NL, c->d_vloc, c->d_vloc_f, vh, vxc);
-  } else {
-    // parts only: Vpsl = 0 into a scratch potential (the second grid)
-    double* pot = (double*)B;
-    hipLaunchKernelGGL(salmon::scf::k_vloc, gr, bl, 0, c->stream, (const cplx<double>*)A, rho, (const double*)nullptr,
-                       xc, g.NL, pot, (float*)nullptr, vh, vxc);
-  }
+  const dim3 bl(256);
+  const int nz = dft::plane_lines(g.NLy), ny = dft::plane_lines(g.NLz);
+  hipLaunchKernelGGL(salmon::scf::k_rho_zy, dim3((g.NLz + nz - 1) / nz, g.NLx), bl, dft::plane_lds(g.NLz, g.NLy), c->stream,
+                     rho, A, g, tw);
+  hipLaunchKernelGGL(salmon::scf::k_coulomb_x, dim3(dft::lines_x_blocks(g)), bl, 0, c->stream, A, g, tw);
+  // parts only: Vpsl = 0 into a scratch potential (the second grid)
+  hipLaunchKernelGGL(salmon::scf::k_vloc_yz, dim3((g.NLy + ny - 1) / ny, g.NLx), bl, dft::plane_lds(g.NLy, g.NLz), c->stream,
+                     (const cplx<double>*)A, g, tw, rho, set_v ? (const double*)c->d_vpsl : (const double*)nullptr, xc,
+                     set_v ? c->d_vloc : (double*)B, set_v ? c->d_vloc_f : (float*)nullptr, vh, vxc);
   LAUNCHCHK(c);
   return SALMON_OK;
 }

@@ -1,63 +1,39 @@
 // Self-consistent local potential of the RT step (ARTED/RT/dt_evolve.f90:
 // 185-207 with no_update_func = 'n'): from the density rho(t+dt), the Hartree
-// potential (ARTED/common/Hartree.f90:20-128: rho(G) by one DFT pass per axis,
-// V_H(G) = 4 pi rho(G)/|G|^2 without G = 0, back by three passes) and the
+// potential (ARTED/common/Hartree.f90:20-128: rho(G), V_H(G) = 4 pi rho(G)/|G|^2
+// without G = 0, and back, in the three launches of dft.hpp) and the
 // PZ81 LDA exchange-correlation potential (src/xc/builtin_pz.f90:24-80 as
 // called by src/xc/salmon_xc.f90:499-511), Vloc = V_H + Vpsl + V_xc.
 // Orthorhombic cells.  FP64 throughout; the complex64 orbitals' potential copy
 // is refreshed from the FP64 one.
 #pragma once
+#include "dft.hpp"
 
 namespace salmon {
 namespace scf {
 
 constexpr int kMaxN = 256;  // points per axis of the DFT passes (twiddle table rows)
 
-// One DFT pass along `axis` over complex rows (one thread per output point):
-// out(l) = sum_m in(m) e^{sgn 2 pi i l m / N}, twiddles tw[axis][j] =
-// (cos, sin)(2 pi j / N) in the order the oracle sums.
-__global__ void __launch_bounds__(256) k_dft_axis(const cplx<double>* __restrict__ in, cplx<double>* __restrict__ out,
-                                                  Grid g, int axis, int sgn, const double* __restrict__ tw) {
-  const int p = blockIdx.x * 256 + threadIdx.x;
-  if (p >= g.NL) return;
-  const int N = axis == 0 ? g.NLx : (axis == 1 ? g.NLy : g.NLz);
-  const int es = axis == 0 ? g.NLy * g.NLz : (axis == 1 ? g.NLz : 1);
-  const int l = (p / es) % N;
-  const int base = p - l * es;
-  const double* t = tw + (size_t)axis * 2 * kMaxN;
-  double re = 0.0, im = 0.0;
-  int j = 0;
-  for (int m = 0; m < N; ++m) {
-    const double c = t[2 * j], s = sgn * t[2 * j + 1];
-    const cplx<double> v = in[base + m * es];
-    re += c * v.re - s * v.im;
-    im += c * v.im + s * v.re;
-    j += l;
-    if (j >= N) j -= N;
-  }
-  out[p] = cplx<double>{re, im};
+// rho(x; y, z) to its z and y transforms.  Grid (blocks of z lines, NLx).
+__global__ void __launch_bounds__(256) k_rho_zy(const double* __restrict__ rho, cplx<double>* __restrict__ f, Grid g,
+                                                const double* __restrict__ tw) {
+  const size_t o = (size_t)blockIdx.y * g.NLy * g.NLz;
+  dft::plane<true>(g.NLz, g.NLy, tw + 4 * kMaxN, tw + 2 * kMaxN, -1.0,
+                   [&](int z, int y) { return cplx<double>{rho[o + y * g.NLz + z], 0.0}; },
+                   [&](int z, int y, cplx<double> v) { f[o + y * g.NLz + z] = v; });
 }
 
-// rho (real) into a complex row
-__global__ void __launch_bounds__(256) k_real_to_cplx(const double* __restrict__ rho, cplx<double>* __restrict__ f,
-                                                      int NL) {
-  const int p = blockIdx.x * 256 + threadIdx.x;
-  if (p < NL) f[p] = cplx<double>{rho[p], 0.0};
-}
-
-// F(G) *= 4 pi / |G|^2 / NL, G = 0 dropped
-__global__ void __launch_bounds__(256) k_coulomb(cplx<double>* __restrict__ F, Grid g) {
-  const int p = blockIdx.x * 256 + threadIdx.x;
-  if (p >= g.NL) return;
-  const int ix = p / (g.NLy * g.NLz), iy = (p / g.NLz) % g.NLy, iz = p % g.NLz;
-  const int nx = ix < g.NLx - g.NLx / 2 ? ix : ix - g.NLx;
-  const int ny = iy < g.NLy - g.NLy / 2 ? iy : iy - g.NLy;
-  const int nz = iz < g.NLz - g.NLz / 2 ? iz : iz - g.NLz;
-  const double pi = 3.141592653589793;
-  const double gx = 2.0 * pi * nx / g.aLx, gy = 2.0 * pi * ny / g.aLy, gz = 2.0 * pi * nz / g.aLz;
-  const double G2 = gx * gx + gy * gy + gz * gz;
-  const double f = (nx == 0 && ny == 0 && nz == 0) ? 0.0 : 4.0 * pi / G2 / g.NL;
-  F[p] = cplx<double>{f * F[p].re, f * F[p].im};
+// The x transform, 4 pi / |G|^2 / NL with G = 0 dropped, and back along x.
+__global__ void __launch_bounds__(256) k_coulomb_x(cplx<double>* __restrict__ f, Grid g, const double* __restrict__ tw) {
+  dft::lines_x(g, f, tw, [&](int ix, int iy, int iz) {
+    const int nx = ix < g.NLx - g.NLx / 2 ? ix : ix - g.NLx;
+    const int ny = iy < g.NLy - g.NLy / 2 ? iy : iy - g.NLy;
+    const int nz = iz < g.NLz - g.NLz / 2 ? iz : iz - g.NLz;
+    const double pi = 3.141592653589793;
+    const double gx = 2.0 * pi * nx / g.aLx, gy = 2.0 * pi * ny / g.aLy, gz = 2.0 * pi * nz / g.aLz;
+    const double G2 = gx * gx + gy * gy + gz * gz;
+    return (nx == 0 && ny == 0 && nz == 0) ? 0.0 : 4.0 * pi / G2 / g.NL;
+  });
 }
 
 // PZ81 e_xc and its density derivative at the total density t (with the
@@ -81,20 +57,25 @@ __device__ __forceinline__ double pz_vxc(double rho) {
   return e + rho * de;
 }
 
-// Vloc = V_H + Vpsl + V_xc into the FP64 potential and its FP32 copy;
-// vh/vxc (nullable) get the parts
-__global__ void __launch_bounds__(256) k_vloc(const cplx<double>* __restrict__ vhc, const double* __restrict__ rho,
-                                              const double* __restrict__ vpsl, int xc, int NL, double* __restrict__ v64,
-                                              float* __restrict__ v32, double* __restrict__ vh, double* __restrict__ vxc) {
-  const int p = blockIdx.x * 256 + threadIdx.x;
-  if (p >= NL) return;
-  const double h = vhc[p].re;
-  const double x = xc ? pz_vxc(rho[p]) : 0.0;
-  const double v = h + (vpsl ? vpsl[p] : 0.0) + x;
-  v64[p] = v;
-  if (v32) v32[p] = (float)v;
-  if (vh) vh[p] = h;
-  if (vxc) vxc[p] = x;
+// V_H from its x-back-transformed rows by the y and z transforms, and Vloc = V_H +
+// Vpsl + V_xc into the FP64 potential and its FP32 copy; vh/vxc (nullable) get the
+// parts.  Grid (blocks of y lines, NLx).
+__global__ void __launch_bounds__(256) k_vloc_yz(const cplx<double>* __restrict__ f, Grid g, const double* __restrict__ tw,
+                                                 const double* __restrict__ rho, const double* __restrict__ vpsl, int xc,
+                                                 double* __restrict__ v64, float* __restrict__ v32,
+                                                 double* __restrict__ vh, double* __restrict__ vxc) {
+  const size_t o = (size_t)blockIdx.y * g.NLy * g.NLz;
+  dft::plane<false>(g.NLy, g.NLz, tw + 2 * kMaxN, tw + 4 * kMaxN, 1.0,
+                    [&](int y, int z) { return f[o + y * g.NLz + z]; },
+                    [&](int y, int z, cplx<double> r) {
+                      const size_t p = o + y * g.NLz + z;
+                      const double h = r.re, x = xc ? pz_vxc(rho[p]) : 0.0;
+                      const double v = h + (vpsl ? vpsl[p] : 0.0) + x;
+                      v64[p] = v;
+                      if (v32) v32[p] = (float)v;
+                      if (vh) vh[p] = h;
+                      if (vxc) vxc[p] = x;
+                    });
 }
 
 // ETRS potential extrapolation (dt_evolve.f90:247-251): Vnew = 3 V - 3 V_old1 +
