@@ -22,32 +22,32 @@ template <typename T>
 struct Sys {
   Grid g;
   KBTables kb;
-  cplx<T>* zu;
-  cplx<T>* h[4];
-  cplx<T>* uv;  // (NKB, Nlma)
-  cplx<T>* ph;  // (NK, NPI) KB phases at this step's midpoint k
-  cplx<T>* phn; // (NK, NPI) KB phases at k + A(t+dt), for the observables
-  cplx<T>* kbv; // (NKB, NT) KB term of every touched point of the current H application
-  const T* vloc;
-  const double* vloc64;
-  const double* kac0;
-  const double* occ;
-  double* rows;  // (NKB, 8)
-  double* rrows; // (kResSteps, NKB, 8), resident kernel
+  gptr<cplx<T>> zu;
+  gptr<cplx<T>> h[4];
+  gptr<cplx<T>> uv;  // (NKB, Nlma)
+  gptr<cplx<T>> ph;  // (NK, NPI) KB phases at this step's midpoint k
+  gptr<cplx<T>> phn; // (NK, NPI) KB phases at k + A(t+dt), for the observables
+  gptr<cplx<T>> kbv; // (NKB, NT) KB term of every touched point of the current H application
+  gptr<const T> vloc;
+  gptr<const double> vloc64;
+  gptr<const double> kac0;
+  gptr<const double> occ;
+  gptr<double> rows;  // (NKB, 8)
+  gptr<double> rrows; // (kResSteps, NKB, 8), resident kernel
   int NK, NB, NKB, zb;
   int sw_zb, sw_tw;          // persistent sweep: column length along z, waves per team
-  const int* kb_order;       // persistent sweep: atoms grouped by colour (no shared grid point within a colour)
-  const int* kb_cstart;      // (ncolor+1) first entry of each colour in kb_order
+  gptr<const int> kb_order;       // persistent sweep: atoms grouped by colour (no shared grid point within a colour)
+  gptr<const int> kb_cstart;      // (ncolor+1) first entry of each colour in kb_order
   int ncolor;
   int pblk, hblk, kblk;      // projection, stencil and KB-apply blocks per orbital
   long first[kPhases + 1];   // first block of the system in each phase
 };
 
 struct Step {
-  const double* ac;  // (nsteps+1, 3), or (nsys, nsteps+1, 3) with ac_stride = 3 (nsteps+1)
-  const int* step;   // device step counter
+  gptr<const double> ac;  // (nsteps+1, 3), or (nsys, nsteps+1, 3) with ac_stride = 3 (nsteps+1)
+  gptr<const int> step;   // device step counter
   double dt;
-  const unsigned short* owner[kPhases];  // system of every block, per phase
+  gptr<const unsigned short> owner[kPhases];  // system of every block, per phase
   long ac_stride;    // doubles between the A(t) tables of consecutive systems (0: one shared table)
   int obs_only;      // persistent sweep: the launch that closes a run (observables only)
 };

@@ -22,25 +22,43 @@ struct Grid {
   double nab[3][5];  // nab(0:4)/H per axis, nab[.][0] unused
 };
 
+// A pointer to device memory kept in a table that kernels read.  The compiler
+// cannot know where a pointer loaded from memory points and would access it with
+// flat instructions, which also count as LDS operations: every wait for LDS, each
+// barrier among them, then waits for the prefetches in flight.
+template <typename T>
+struct gptr {
+  T* p;
+  gptr() = default;
+  __host__ __device__ gptr(T* q) : p(q) {}
+  __host__ __device__ operator T*() const {
+#ifdef __HIP_DEVICE_COMPILE__
+    return (T*)(__attribute__((address_space(1))) T*)(uintptr_t)p;  // (via an integer: a cast there and back folds away)
+#else
+    return p;
+#endif
+  }
+};
+
 // Kleinman-Bylander tables in device memory.  "Packed" indices enumerate the
 // sphere points of all atoms one atom after another (the reference's NPI
 // vector, opt_variables.f90:233-265).
 struct KBTables {
   int NI, Nps, Nlma, NPI, NT, NE;
-  const int* atom_start;  // (NI+1) packed offset of each atom's sphere
-  const int* pidx;        // (NPI) 0-based grid index of each packed point
-  const double* pos;      // (NPI*3) unwrapped coordinates Lx*Hx - Jxx*aLx, ...
-  const int* lma_atom;    // (Nlma) 0-based atom of each projector
-  const int* atom_lma;    // (NI+1) first projector of each atom (projectors grouped by atom)
+  gptr<const int> atom_start;  // (NI+1) packed offset of each atom's sphere
+  gptr<const int> pidx;        // (NPI) 0-based grid index of each packed point
+  gptr<const double> pos;      // (NPI*3) unwrapped coordinates Lx*Hx - Jxx*aLx, ...
+  gptr<const int> lma_atom;    // (Nlma) 0-based atom of each projector
+  gptr<const int> atom_lma;    // (NI+1) first projector of each atom (projectors grouped by atom)
   int max_lpa;            // most projectors of one atom
-  const double* lma_sign; // (Nlma) iuV as a real
-  const double* uv;       // (Nlma*Nps) uV(j,ilma) at [ilma*Nps + j]
-  const int* pt2t;        // (NL) touched-point number of a grid point, or -1
-  const int* t_start;     // (NT+1) first entry of each touched point
-  const int* e_lma;       // (NE) projector of each entry
-  const int* e_jp;        // (NE) packed point of each entry
-  const int* tj_start;    // (NT+1) first packed point of each touched point
-  const int* tj;          // the touched points' packed points, of atoms with projectors
+  gptr<const double> lma_sign; // (Nlma) iuV as a real
+  gptr<const double> uv;       // (Nlma*Nps) uV(j,ilma) at [ilma*Nps + j]
+  gptr<const int> pt2t;        // (NL) touched-point number of a grid point, or -1
+  gptr<const int> t_start;     // (NT+1) first entry of each touched point
+  gptr<const int> e_lma;       // (NE) projector of each entry
+  gptr<const int> e_jp;        // (NE) packed point of each entry
+  gptr<const int> tj_start;    // (NT+1) first packed point of each touched point
+  gptr<const int> tj;          // the touched points' packed points, of atoms with projectors
 };
 
 constexpr int kWave = 64;

@@ -90,21 +90,26 @@ __global__ void __launch_bounds__(256) k_gsb_overlap(GsBlock b, int j0, int np) 
   const bool oka = ia < ni, okb = li < np;
   const int p0 = c * b.chunk, p1 = min(b.NL, p0 + b.chunk);
   f64x4 cr = {0, 0, 0, 0}, ci = cr;
-  for (int q = p0 + wv * 16; q < p1; q += 64) {
-    cplx<double> x[4], y[4];
+  // two groups of 16 points with their loads in flight together: the loop's time
+  // is their latency
+  for (int q = p0 + wv * 16; q < p1; q += 128) {
+    cplx<double> x[8], y[8];
 #pragma unroll
-    for (int s = 0; s < 4; ++s) {
-      const int p = q + 4 * s + lg, pc = min(p, p1 - 1);
+    for (int s = 0; s < 8; ++s) {
+      const int p = q + (s & 4) * 16 + 4 * (s & 3) + lg, pc = min(p, p1 - 1);
       x[s] = A[pc];
       y[s] = P[pc];
-      const bool ok = p < p1;
+    }
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+      const bool ok = q + (s & 4) * 16 + 4 * (s & 3) + lg < p1;
       x[s].re = ok && oka ? x[s].re : 0.0;
       x[s].im = ok && oka ? x[s].im : 0.0;
       y[s].re = ok && okb ? y[s].re : 0.0;
       y[s].im = ok && okb ? y[s].im : 0.0;
     }
 #pragma unroll
-    for (int s = 0; s < 4; ++s) {
+    for (int s = 0; s < 8; ++s) {
       cr = mfma_f64(x[s].re, y[s].re, cr);
       ci = mfma_f64(x[s].re, y[s].im, ci);
       cr = mfma_f64(x[s].im, y[s].im, cr);
@@ -131,35 +136,51 @@ __global__ void __launch_bounds__(256) k_gsb_overlap(GsBlock b, int j0, int np) 
   {
     const cplx<double>* q = b.part + ((size_t)k * b.ntile + tile) * b.nchunk * 256 + t;
     double sr = 0.0, si = 0.0;
-#pragma unroll 8
-    for (int e = 0; e < b.nchunk; ++e) {
-      const cplx<double> v = load_agent(q + (size_t)e * 256);
-      sr += v.re;
-      si += v.im;
+    for (int e0 = 0; e0 < b.nchunk; e0 += 16) {  // 16 loads in flight, clamped
+      cplx<double> v[16];
+#pragma unroll
+      for (int e = 0; e < 16; ++e) v[e] = load_agent(q + (size_t)min(e0 + e, b.nchunk - 1) * 256);
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        sr = e0 + e < b.nchunk ? sr + v[e].re : sr;
+        si = e0 + e < b.nchunk ? si + v[e].im : si;
+      }
     }
     const int i = tile * 16 + t / 16;
     if (i < b.NB) store_agent(&b.C[((size_t)k * b.NB + i) * 16 + (t & 15)], cplx<double>{sr * b.Hxyz, si * b.Hxyz});
   }
   if (!arrive_last(cnt, nt)) return;
-  // the last tile's block: G - C^H C, its Cholesky factor and inverse, W
-  __shared__ cplx<double> G[16][17], R[16][17];
+  // the last tile's block: G - C^H C, its Cholesky factor and inverse, W.  C comes
+  // in tiles of 16 bands, a value per thread, the next one while one is used.
+  __shared__ cplx<double> G[16][17], R[16][17], Ct[16][17];
   __shared__ int bad;
   const int row = t / 16, col = t & 15;
-  const cplx<double>* C = b.C + (size_t)k * b.NB * 16;
+  const cplx<double>* C = b.C + (size_t)k * b.NB * 16 + row * 16 + col;
+  auto next = [&](int i) { return load_agent(C + (size_t)min(i, j0 - 16) * 16); };  // (j0: whole panels)
   if (t == 0) bad = 0;
   double g0 = 0.0;  // the band's squared norm before
   {
-    cplx<double> v{row == col ? 1.0 : 0.0, 0.0};
+    cplx<double> v{row == col ? 1.0 : 0.0, 0.0}, ct{0, 0};
+    if (j0 > 0) ct = next(0);
     if (row < np && col < np) {
-      v = load_agent(&C[(size_t)(j0 + row) * 16 + col]);
+      v = load_agent(C + (size_t)j0 * 16);
       if (row == col) g0 = v.re;
-      for (int i = 0; i < j0; ++i) {
-        const cplx<double> x = load_agent(&C[(size_t)i * 16 + row]), y = load_agent(&C[(size_t)i * 16 + col]);
-        v.re -= x.re * y.re + x.im * y.im;
-        v.im -= x.re * y.im - x.im * y.re;
-      }
     } else if (row == col) {
       g0 = 1.0;
+    }
+    for (int i0 = 0; i0 < j0; i0 += 16) {
+      Ct[row][col] = ct;
+      __syncthreads();
+      ct = next(i0 + 16);
+      if (row < np && col < np) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          const cplx<double> x = Ct[i][row], y = Ct[i][col];
+          v.re -= x.re * y.re + x.im * y.im;
+          v.im -= x.re * y.im - x.im * y.re;
+        }
+      }
+      __syncthreads();
     }
     G[row][col] = v;
     R[row][col] = cplx<double>{row == col ? 1.0 : 0.0, 0.0};
@@ -192,14 +213,21 @@ __global__ void __launch_bounds__(256) k_gsb_overlap(GsBlock b, int j0, int np) 
     return;
   }
   cplx<double>* W = b.W + (size_t)k * b.NB * 16;
-  for (int i = row; i < j0; i += 16) {  // -C R^-1
+  cplx<double> ct{0, 0};
+  if (j0 > 0) ct = next(0);
+  for (int i0 = 0; i0 < j0; i0 += 16) {  // -C R^-1
+    Ct[row][col] = ct;
+    __syncthreads();
+    ct = next(i0 + 16);
     cplx<double> v{0, 0};
-    for (int m = 0; m <= col; ++m) {
-      const cplx<double> x = load_agent(&C[(size_t)i * 16 + m]), y = R[m][col];
+#pragma unroll
+    for (int m = 0; m < 16; ++m) {
+      const cplx<double> x = Ct[row][m], y = R[m][col];  // (zero for m > col)
       v.re -= x.re * y.re - x.im * y.im;
       v.im -= x.re * y.im + x.im * y.re;
     }
-    W[(size_t)i * 16 + col] = v;
+    W[(size_t)(i0 + row) * 16 + col] = v;
+    __syncthreads();
   }
   if (row < np) W[(size_t)(j0 + row) * 16 + col] = R[row][col];
 }

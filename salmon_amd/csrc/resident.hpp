@@ -55,12 +55,12 @@ inline size_t res_lds(const Grid& g, int NPI, int NI) {
 
 // Per-system tables of the resident kernel.
 struct ResTab {
-  const int* prim;      // (NL) first sphere point covering a grid point, or NPI
-  const int* code;      // (NPI) px | py << 10 | pz << 20 into the per-axis phase tables
-  const double* uvp;    // (NPI, kResLpa) uV(j, l) of the sphere point's atom, zero past its projectors
-  const double* sgp;    // (NI, kResLpa) iuV
-  const int* ov_start;  // (nov+1) grid points inside several spheres: entries
-  const int* ov_jp;     // [ov_start[o]+1, ov_start[o+1]) of ov_jp add into ov_jp[ov_start[o]]
+  gptr<const int> prim;      // (NL) first sphere point covering a grid point, or NPI
+  gptr<const int> code;      // (NPI) px | py << 10 | pz << 20 into the per-axis phase tables
+  gptr<const double> uvp;    // (NPI, kResLpa) uV(j, l) of the sphere point's atom, zero past its projectors
+  gptr<const double> sgp;    // (NI, kResLpa) iuV
+  gptr<const int> ov_start;  // (nov+1) grid points inside several spheres: entries
+  gptr<const int> ov_jp;     // [ov_start[o]+1, ov_start[o+1]) of ov_jp add into ov_jp[ov_start[o]]
   int nov;
   double cc[3][4], dc[3][4];  // -lap(n)/2 and nab(n) per axis, n = 1..4
 };
