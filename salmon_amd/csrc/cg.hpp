@@ -355,8 +355,14 @@ __global__ void __launch_bounds__(kWide) k_cg_sub(State S, const cplx<double>* _
                                                 int role, int it, int ncg) {
   const int k = blockIdx.y;
   const int skip = role != SUB_START ? S.done[k] : 0;
-  const int c = blockIdx.x, t = threadIdx.x & (kSubPts - 1);
+  // consecutive blocks go to consecutive ones of the eight dies: the die of a
+  // projection block's kChunk points also takes the two blocks here that hold them,
+  // and finds the lower bands in its L2 cache
+  int c = blockIdx.x;
+  if ((c | 15) < S.nsub) c = (c & ~15) | (c & 7) << 1 | (c >> 3 & 1);
+  const int t = threadIdx.x & (kSubPts - 1);
   const int part = __builtin_amdgcn_readfirstlane(threadIdx.x / kSubPts);
+  static_assert(kChunk == 2 * kSubPts, "two subtraction blocks per projection block");
   const size_t off = (size_t)k * S.NL;
   const double xhx = S.sc[k * kNS + XHX];
   const cplx<double>* B = zu + (size_t)k * S.NB * S.NL;
