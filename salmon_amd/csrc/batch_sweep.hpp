@@ -160,9 +160,13 @@ __device__ __forceinline__ void col_sweep(const Grid& g, bool act, int tl, cplx<
     const int Xs = wrap_once(X, NLx);
     load_run<T, ZB>(in + (size_t)Xs * P + w0, d);
   };
-  // per-point operands, double-buffered by plane parity
-  T V[2][ZB];
-  cplx<T> zz[2][ZB], a0[2][ZB], a1[2][ZB];
+  // per-point operands: complex64, of the plane, loaded at the start of its step;
+  // FP64, double-buffered by plane parity and loaded a step ahead (there the
+  // compiler spills more with one buffer: 32^3 x 2048 2.39 and 2.52 ms a step)
+  constexpr bool kAhead = sizeof(T) == 4;
+  constexpr int OB = kAhead ? 1 : 2;
+  T V[OB][ZB];
+  cplx<T> zz[OB][ZB], a0[OB][ZB], a1[OB][ZB];
   auto ld_ops = [&](int X, int b) {
     const size_t pb = (size_t)X * P + w0;
 #pragma unroll
@@ -175,7 +179,7 @@ __device__ __forceinline__ void col_sweep(const Grid& g, bool act, int tl, cplx<
   };
   // every thread loads (threads without a column from a valid point of the
   // orbital) so that no branch separates the loads from their uses
-  ld_ops(0, 0);
+  if constexpr (!kAhead) ld_ops(0, 0);
 #pragma unroll
   for (int X = -4; X <= 4; ++X) ld(X, win[(X + kColWin) % kColWin]);
   for (int x0 = 0; x0 < NLx; x0 += kColWin) {
@@ -185,10 +189,11 @@ __device__ __forceinline__ void col_sweep(const Grid& g, bool act, int tl, cplx<
       if (x >= NLx) break;
       const size_t pb = (size_t)x * P + w0;
       const int soff = col ? (int)(pb * sizeof(cplx<T>)) : kDropOffset;
-      const int cb = j & 1;  // operand buffer of plane x (x0 is even)
-      ld_ops(x + 1 < NLx ? x + 1 : 0, cb ^ 1);
+      const int cb = kAhead ? 0 : j & 1;  // operand buffer of plane x (x0 is even)
+      if constexpr (kAhead) ld_ops(x, 0);
+      else ld_ops(x + 1 < NLx ? x + 1 : 0, cb ^ 1);
       ld(x + 5, win[(j + 5) % kColWin]);
-      cplx<T>* pln = pl + cb * PS;
+      cplx<T>* pln = pl + (j & 1) * PS;
 #pragma unroll
       for (int q = 0; q < ZB; ++q) pln[own + q] = win[j][q];
       lds_barrier();
@@ -203,70 +208,81 @@ __device__ __forceinline__ void col_sweep(const Grid& g, bool act, int tl, cplx<
       for (int q = 0; q < ZB; ++q) zw[4 + q] = win[j][q];
       // per point: L (vr, vi), the k term sum_a k_a G_a (wr, wi), the
       // observables' sums from L and each G_a as its axis completes
-      T vr[ZB], vi[ZB], wr[ZB], wi[ZB];
+      T vr[ZB], vi[ZB], wr[ZB], wi[ZB], gr[ZB], gi[ZB];
       double er[ZB], ei[ZB];
 #pragma unroll
       for (int q = 0; q < ZB; ++q) {
         // threads without a column add zeros to the observables
         er[q] = col ? (double)win[j][q].re : 0.0;
         ei[q] = col ? (double)win[j][q].im : 0.0;
-        T gr = 0, gi = 0;
-        vr[q] = vi[q] = 0;
-#pragma unroll
-        for (int n = 1; n <= 4; ++n) {
-          const cplx<T> ep = zw[4 + q + n], em = zw[4 + q - n];
-          vr[q] += C[2][n] * (ep.re + em.re);
-          vi[q] += C[2][n] * (ep.im + em.im);
-          gr += D[2][n] * (ep.re - em.re);
-          gi += D[2][n] * (ep.im - em.im);
-        }
-        wr[q] = kt[2] * gr;
-        wi[q] = kt[2] * gi;
-        if constexpr (MODE >= 2) acc[5] += er[q] * (double)gi - ei[q] * (double)gr;
+        vr[q] = vi[q] = wr[q] = wi[q] = gr[q] = gi[q] = 0;
       }
-      {
-        T gr[ZB], gi[ZB];
-#pragma unroll
-        for (int q = 0; q < ZB; ++q) gr[q] = gi[q] = 0;
-#pragma unroll
-        for (int n = 1; n <= 4; ++n) {
-#pragma unroll
-          for (int q = 0; q < ZB; ++q) {
-            const cplx<T> ep = pln[yo[n - 1] + q], em = pln[yo[3 + n] + q];
-            vr[q] += C[1][n] * (ep.re + em.re);
-            vi[q] += C[1][n] * (ep.im + em.im);
-            gr[q] += D[1][n] * (ep.re - em.re);
-            gi[q] += D[1][n] * (ep.im - em.im);
-          }
-        }
+      auto add = [&](int a, int n, int q, const cplx<T>& ep, const cplx<T>& em) __attribute__((always_inline)) {
+        vr[q] += C[a][n] * (ep.re + em.re);
+        vi[q] += C[a][n] * (ep.im + em.im);
+        gr[q] += D[a][n] * (ep.re - em.re);
+        gi[q] += D[a][n] * (ep.im - em.im);
+      };
+      auto axis_done = [&](int a) __attribute__((always_inline)) {
 #pragma unroll
         for (int q = 0; q < ZB; ++q) {
-          wr[q] += kt[1] * gr[q];
-          wi[q] += kt[1] * gi[q];
-          if constexpr (MODE >= 2) acc[4] += er[q] * (double)gi[q] - ei[q] * (double)gr[q];
+          wr[q] += kt[a] * gr[q];
+          wi[q] += kt[a] * gi[q];
+          if constexpr (MODE >= 2) acc[3 + a] += er[q] * (double)gi[q] - ei[q] * (double)gr[q];
+          gr[q] = gi[q] = 0;
         }
-      }
-      {
-        T gr[ZB], gi[ZB];
+      };
+      auto add_x = [&]() __attribute__((always_inline)) {
 #pragma unroll
-        for (int q = 0; q < ZB; ++q) gr[q] = gi[q] = 0;
+        for (int n = 1; n <= 4; ++n)
 #pragma unroll
-        for (int n = 1; n <= 4; ++n) {
+          for (int q = 0; q < ZB; ++q) add(0, n, q, win[(j + n) % kColWin][q], win[(j + kColWin - n) % kColWin][q]);
+        axis_done(0);
+      };
+      auto add_z = [&]() __attribute__((always_inline)) {
 #pragma unroll
-          for (int q = 0; q < ZB; ++q) {
-            const cplx<T> ep = win[(j + n) % kColWin][q], em = win[(j + kColWin - n) % kColWin][q];
-            vr[q] += C[0][n] * (ep.re + em.re);
-            vi[q] += C[0][n] * (ep.im + em.im);
-            gr[q] += D[0][n] * (ep.re - em.re);
-            gi[q] += D[0][n] * (ep.im - em.im);
-          }
-        }
+        for (int q = 0; q < ZB; ++q)
+#pragma unroll
+          for (int n = 1; n <= 4; ++n) add(2, n, q, zw[4 + q + n], zw[4 + q - n]);
+        axis_done(2);
+      };
+      cplx<T> yp[2][ZB], ym[2][ZB];
+      auto ld_y = [&](int n) __attribute__((always_inline)) {
 #pragma unroll
         for (int q = 0; q < ZB; ++q) {
-          wr[q] += kt[0] * gr[q];
-          wi[q] += kt[0] * gi[q];
-          if constexpr (MODE >= 2) acc[3] += er[q] * (double)gi[q] - ei[q] * (double)gr[q];
+          yp[n & 1][q] = pln[yo[n - 1] + q];
+          ym[n & 1][q] = pln[yo[3 + n] + q];
         }
+      };
+      if constexpr (kAhead) {
+        // The LDS reads go out one stage of arithmetic ahead of their use: the z
+        // window before the x terms, which need none, each pair of y runs before
+        // the terms of the last.  The fences keep the compiler from moving them
+        // back to their use, where each of nine waits showed: 20x20x28 x 276 step
+        // launches 190 -> 176 us.  FP64 has no registers for it (0.81 times as fast).
+        __builtin_amdgcn_sched_barrier(0);
+        add_x();
+        ld_y(1);
+        __builtin_amdgcn_sched_barrier(0);
+        add_z();
+#pragma unroll
+        for (int n = 1; n <= 4; ++n) {
+          if (n < 4) ld_y(n + 1);
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int q = 0; q < ZB; ++q) add(1, n, q, yp[n & 1][q], ym[n & 1][q]);
+        }
+        axis_done(1);
+      } else {
+        add_z();
+#pragma unroll
+        for (int n = 1; n <= 4; ++n) {
+          ld_y(n);
+#pragma unroll
+          for (int q = 0; q < ZB; ++q) add(1, n, q, yp[n & 1][q], ym[n & 1][q]);
+        }
+        axis_done(1);
+        add_x();
       }
       if constexpr (MODE >= 2) {
 #pragma unroll

@@ -22,22 +22,25 @@ struct Grid {
   double nab[3][5];  // nab(0:4)/H per axis, nab[.][0] unused
 };
 
-// A pointer to device memory kept in a table that kernels read.  The compiler
-// cannot know where a pointer loaded from memory points and would access it with
-// flat instructions, which also count as LDS operations: every wait for LDS, each
-// barrier among them, then waits for the prefetches in flight.
+// A pointer that is known to point to device memory.  The compiler cannot see
+// that of one loaded from a table and would access it with flat instructions, which also count as LDS operations: every wait
+// for LDS, each barrier among them, then waits for the loads in flight.
+template <typename T>
+__host__ __device__ __forceinline__ T* as_global(T* p) {
+#ifdef __HIP_DEVICE_COMPILE__
+  return (T*)(__attribute__((address_space(1))) T*)(uintptr_t)p;  // (via an integer: a cast there and back folds away)
+#else
+  return p;
+#endif
+}
+
+// Such a pointer kept in a table that kernels read.
 template <typename T>
 struct gptr {
   T* p;
   gptr() = default;
   __host__ __device__ gptr(T* q) : p(q) {}
-  __host__ __device__ operator T*() const {
-#ifdef __HIP_DEVICE_COMPILE__
-    return (T*)(__attribute__((address_space(1))) T*)(uintptr_t)p;  // (via an integer: a cast there and back folds away)
-#else
-    return p;
-#endif
-  }
+  __host__ __device__ operator T*() const { return as_global(p); }
 };
 
 // Kleinman-Bylander tables in device memory.  "Packed" indices enumerate the
