@@ -94,7 +94,7 @@ __global__ void __launch_bounds__(256) k_b_project(const Sys<T>* __restrict__ S,
 // orbitals entering step n (persistent sweep; at the end of a run n = nsteps,
 // the last row of the A table).
 template <typename T>
-__global__ void __launch_bounds__(256) k_b_phase(const Sys<T>* __restrict__ S, Step st, int which) {
+__device__ __forceinline__ void phase_value(const Sys<T>* __restrict__ S, const Step& st, int which) {
   const Sys<T>& y = S[blockIdx.y];
   const long i = (long)blockIdx.x * 256 + threadIdx.x;
   if (i >= (long)y.NK * y.kb.NPI) return;
@@ -110,6 +110,21 @@ __global__ void __launch_bounds__(256) k_b_phase(const Sys<T>* __restrict__ S, S
   double s, c;
   sincos(kx * y.kb.pos[3 * jp] + ky * y.kb.pos[3 * jp + 1] + kz * y.kb.pos[3 * jp + 2], &s, &c);
   (which ? y.phn : y.ph)[i] = cplx<T>{(T)c, (T)s};
+}
+
+template <typename T>
+__global__ void __launch_bounds__(256) k_b_phase(const Sys<T>* __restrict__ S, Step st, int which) {
+  phase_value<T>(S, st, which);
+}
+
+// What a launch of the persistent sweep finds done: the phases it uses (`which`;
+// with a second grid layer also those of which = 2) and its work queue at zero.
+// One launch instead of three of 4 to 5 us each beside a step of 20x20x28 x 276
+// orbitals of 180.
+template <typename T>
+__global__ void __launch_bounds__(256) k_b_begin(const Sys<T>* __restrict__ S, Step st, int which, int* next) {
+  if (threadIdx.x == 0 && blockIdx.x + blockIdx.y + blockIdx.z == 0) *next = 0;
+  phase_value<T>(S, st, blockIdx.z ? 2 : which);
 }
 
 // KB term of every touched grid point of every orbital (pseudo_pt phase 2,
@@ -312,27 +327,32 @@ __global__ void __launch_bounds__(256) k_b_observe(const Sys<T>* __restrict__ S,
 // Per-system sums of the rows (one block per system) into res(n - lag, s, 0..7),
 // n the device step counter (lag 1: the rows hold the previous step's
 // observables; nothing before the first step).
+// tick: the block that finishes last moves the step counter on (arrive: zero
+// between launches).
 template <typename T>
 __global__ void __launch_bounds__(256) k_b_sum(const Sys<T>* __restrict__ S, int nsys, int* step, double* res,
-                                               int lag) {
+                                               int lag, int tick, unsigned* arrive) {
   __shared__ double smem[4 * 8];
-  if (*step - lag < 0) return;
-  const Sys<T>& y = S[blockIdx.x];
-  double v[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-  for (int r = threadIdx.x; r < y.NKB; r += 256) {
+  const int now = *step, n = now - lag;
+  if (n >= 0) {
+    const Sys<T>& y = S[blockIdx.x];
+    double v[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    for (int r = threadIdx.x; r < y.NKB; r += 256) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) v[i] += y.rows[(size_t)r * 8 + i];
-  }
-  block_sum256<8>(v, smem);
-  if (threadIdx.x == 0) {
-    const int n = *step - lag;
+      for (int i = 0; i < 8; ++i) v[i] += y.rows[(size_t)r * 8 + i];
+    }
+    block_sum256<8>(v, smem);
+    if (threadIdx.x == 0) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) res[((size_t)n * nsys + blockIdx.x) * 8 + i] = v[i];
+      for (int i = 0; i < 8; ++i) res[((size_t)n * nsys + blockIdx.x) * 8 + i] = v[i];
+    }
   }
-}
-
-__global__ void k_b_tick(int* step) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) *step += 1;
+  if (!tick) return;
+  __syncthreads();  // the block's threads have read the counter
+  if (threadIdx.x == 0 && agent_arrive(arrive) == gridDim.x - 1) {
+    *arrive = 0;
+    *step = now + 1;
+  }
 }
 
 }  // namespace batch

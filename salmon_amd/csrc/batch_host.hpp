@@ -35,7 +35,7 @@ struct salmon_batch {
   bool sweep = false;
   int2* d_items = nullptr;        // (system, first orbital), costliest first (in bufs)
   int nitems = 0;
-  int* d_next = nullptr;          // work counter of the sweep launch
+  int* d_next = nullptr;          // work counter of the sweep launch; arrivals of the sums' blocks
   // batches of systems whose orbitals fit in LDS (resident.hpp): one launch per
   // workgroup shape (device memory in bufs)
   struct ResClass {
@@ -356,8 +356,6 @@ static int sweep_plan(salmon_batch* b, std::vector<Sys<T>>& S) {
     return bfail(b, SALMON_ERR_NOMEM, "batch work list");
   b->bufs.push_back(b->d_items);
   BHIP(b, hipMemcpy(b->d_items, it.data(), sizeof(int2) * it.size(), hipMemcpyHostToDevice));
-  if (!b->d_next) BHIP(b, hipMalloc((void**)&b->d_next, sizeof(int)));
-  BHIP(b, hipMemset(b->d_next, 0, sizeof(int)));
   int dev = 0, ncu = 0, per = 0;
   BHIP(b, hipGetDevice(&dev));
   BHIP(b, hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
@@ -465,6 +463,10 @@ static int batch_build(salmon_batch* b) {
     b->bufs.push_back(b->d_owner[ph]);
     BHIP(b, hipMemcpy(b->d_owner[ph], own.data(), sizeof(unsigned short) * own.size(), hipMemcpyHostToDevice));
   }
+  if (!b->d_next) {
+    BHIP(b, hipMalloc((void**)&b->d_next, 2 * sizeof(int)));
+    BHIP(b, hipMemset(b->d_next, 0, 2 * sizeof(int)));
+  }
   b->sweep = b->resident;
   if (!b->resident && (r = sweep_plan<T>(b, S))) return r;
   if (hipMalloc(&b->d_sys, sizeof(Sys<T>) * n) != hipSuccess) return bfail(b, SALMON_ERR_NOMEM, "batch descriptors");
@@ -472,6 +474,20 @@ static int batch_build(salmon_batch* b) {
   BHIP(b, hipMemcpy(b->d_sys, S.data(), sizeof(Sys<T>) * n, hipMemcpyHostToDevice));
   b->ready = true;
   return SALMON_OK;
+}
+
+// One launch of the persistent sweep, its phases (`which`, see k_b_phase; layers = 2:
+// also those of which = 2) and work queue before it.
+template <typename T>
+static void batch_sweep_launch(salmon_batch* b, const Sys<T>* S, const Step& st, int which, int layers) {
+  hipLaunchKernelGGL(k_b_begin<T>, dim3((unsigned)std::max(1L, (b->max_ph + 255) / 256), (unsigned)b->ctx.size(), layers),
+                     dim3(256), 0, b->stream, S, st, which, b->d_next);
+  if constexpr (sizeof(T) == 4)
+    hipLaunchKernelGGL((k_b_sweep<T, 4>), dim3(b->sweep_grid), dim3(sweep_waves<T>() * kWave), b->sweep_lds, b->stream,
+                       S, st, (const int2*)b->d_items, b->nitems, b->d_next);
+  else
+    hipLaunchKernelGGL((k_b_sweep<T, 2>), dim3(b->sweep_grid), dim3(sweep_waves<T>() * kWave), b->sweep_lds, b->stream,
+                       S, st, (const int2*)b->d_items, b->nitems, b->d_next);
 }
 
 // One step's launches (captured by batch_run).
@@ -484,19 +500,9 @@ static int batch_enqueue_step(salmon_batch* b, double dt, long ac_stride) {
   if (b->sweep) {
     // the step's launch also forms the previous step's observables (at
     // A(t_n)), whose rows the sum then takes
-    if (b->max_ph > 0) {
-      hipLaunchKernelGGL(k_b_phase<T>, dim3((unsigned)((b->max_ph + 255) / 256), n), dim3(256), 0, b->stream, S, st, 0);
-      hipLaunchKernelGGL(k_b_phase<T>, dim3((unsigned)((b->max_ph + 255) / 256), n), dim3(256), 0, b->stream, S, st, 2);
-    }
-    hipLaunchKernelGGL(k_b_qreset, dim3(1), dim3(64), 0, b->stream, b->d_next);
-    if constexpr (sizeof(T) == 4)
-      hipLaunchKernelGGL((k_b_sweep<T, 4>), dim3(b->sweep_grid), dim3(sweep_waves<T>() * kWave), b->sweep_lds, b->stream, S, st,
-                         (const int2*)b->d_items, b->nitems, b->d_next);
-    else
-      hipLaunchKernelGGL((k_b_sweep<T, 2>), dim3(b->sweep_grid), dim3(sweep_waves<T>() * kWave), b->sweep_lds, b->stream, S, st,
-                         (const int2*)b->d_items, b->nitems, b->d_next);
-    hipLaunchKernelGGL(k_b_sum<T>, dim3(n), dim3(256), 0, b->stream, S, n, b->d_step, b->d_res, 1);
-    hipLaunchKernelGGL(k_b_tick, dim3(1), dim3(64), 0, b->stream, b->d_step);
+    batch_sweep_launch<T>(b, S, st, 0, 2);
+    hipLaunchKernelGGL(k_b_sum<T>, dim3(n), dim3(256), 0, b->stream, S, n, b->d_step, b->d_res, 1, 1,
+                       (unsigned*)b->d_next + 1);
     BHIP(b, hipGetLastError());
     return SALMON_OK;
   }
@@ -516,8 +522,8 @@ static int batch_enqueue_step(salmon_batch* b, double dt, long ac_stride) {
   if (b->max_ph > 0)
     hipLaunchKernelGGL(k_b_phase<T>, dim3((unsigned)((b->max_ph + 255) / 256), n), dim3(256), 0, b->stream, S, st, 1);
   hipLaunchKernelGGL(k_b_observe<T>, dim3((unsigned)b->first[3][0]), dim3(256), 0, b->stream, S, n, st);
-  hipLaunchKernelGGL(k_b_sum<T>, dim3(n), dim3(256), 0, b->stream, S, n, b->d_step, b->d_res, 0);
-  hipLaunchKernelGGL(k_b_tick, dim3(1), dim3(64), 0, b->stream, b->d_step);
+  hipLaunchKernelGGL(k_b_sum<T>, dim3(n), dim3(256), 0, b->stream, S, n, b->d_step, b->d_res, 0, 1,
+                     (unsigned*)b->d_next + 1);
   BHIP(b, hipGetLastError());
   return SALMON_OK;
 }
@@ -554,16 +560,6 @@ static int batch_k_descriptors(salmon_batch* b, const double* const* kbase) {
   return SALMON_OK;
 }
 
-template <typename T>
-static void batch_sweep_launch(salmon_batch* b, const Sys<T>* S, const Step& st) {
-  if constexpr (sizeof(T) == 4)
-    hipLaunchKernelGGL((k_b_sweep<T, 4>), dim3(b->sweep_grid), dim3(sweep_waves<T>() * kWave), b->sweep_lds, b->stream,
-                       S, st, (const int2*)b->d_items, b->nitems, b->d_next);
-  else
-    hipLaunchKernelGGL((k_b_sweep<T, 2>), dim3(b->sweep_grid), dim3(sweep_waves<T>() * kWave), b->sweep_lds, b->stream,
-                       S, st, (const int2*)b->d_items, b->nitems, b->d_next);
-}
-
 // One Taylor-4 step (hamiltonian.f90:27-123) of every orbital of the batch at
 // the k points kbase[i] over dt, without observables: the persistent sweep
 // with the step counter at 0 (so no observables are formed) and A = 0.
@@ -576,10 +572,7 @@ static int batch_taylor(salmon_batch* b, const double* const* kbase, double dt) 
   if (b->resident) return resident_launch<T>(b, S, ResArgs{nullptr, 0L, 0, 1, dt, 1, 0}, nullptr);
   const Step st{b->d_zero_ac, b->d_zero_step, dt,
                 {b->d_owner[0], b->d_owner[1], b->d_owner[2], b->d_owner[3], b->d_owner[4]}, 0L};
-  if (b->max_ph > 0)
-    hipLaunchKernelGGL(k_b_phase<T>, dim3((unsigned)((b->max_ph + 255) / 256), n), dim3(256), 0, b->stream, S, st, 0);
-  hipLaunchKernelGGL(k_b_qreset, dim3(1), dim3(64), 0, b->stream, b->d_next);
-  batch_sweep_launch<T>(b, S, st);
+  batch_sweep_launch<T>(b, S, st, 0, 1);
   BHIP(b, hipGetLastError());
   return SALMON_OK;
 }
@@ -606,11 +599,9 @@ static int batch_observe(salmon_batch* b, const double* const* kbase, double* ou
   } else {
     const Step st{b->d_zero_ac, b->d_zero_step, 0.0,
                   {b->d_owner[0], b->d_owner[1], b->d_owner[2], b->d_owner[3], b->d_owner[4]}, 0L, 1};
-    if (b->max_ph > 0)
-      hipLaunchKernelGGL(k_b_phase<T>, dim3((unsigned)((b->max_ph + 255) / 256), n), dim3(256), 0, b->stream, S, st, 2);
-    hipLaunchKernelGGL(k_b_qreset, dim3(1), dim3(64), 0, b->stream, b->d_next);
-    batch_sweep_launch<T>(b, S, st);
-    hipLaunchKernelGGL(k_b_sum<T>, dim3(n), dim3(256), 0, b->stream, S, n, b->d_zero_step, b->d_res, 0);
+    batch_sweep_launch<T>(b, S, st, 2, 1);
+    hipLaunchKernelGGL(k_b_sum<T>, dim3(n), dim3(256), 0, b->stream, S, n, b->d_zero_step, b->d_res, 0, 0,
+                       (unsigned*)nullptr);
     BHIP(b, hipGetLastError());
   }
   BHIP(b, hipMemcpyAsync(out, b->d_res, sizeof(double) * 8 * (size_t)n, hipMemcpyDeviceToHost, b->stream));
@@ -627,16 +618,8 @@ static int batch_close_sweep(salmon_batch* b, double dt, long ac_stride) {
   const Sys<T>* S = (const Sys<T>*)b->d_sys;
   const Step st{b->d_ac, b->d_step, dt, {b->d_owner[0], b->d_owner[1], b->d_owner[2], b->d_owner[3], b->d_owner[4]},
                 ac_stride, 1};
-  if (b->max_ph > 0)
-    hipLaunchKernelGGL(k_b_phase<T>, dim3((unsigned)((b->max_ph + 255) / 256), n), dim3(256), 0, b->stream, S, st, 2);
-  hipLaunchKernelGGL(k_b_qreset, dim3(1), dim3(64), 0, b->stream, b->d_next);
-  if constexpr (sizeof(T) == 4)
-    hipLaunchKernelGGL((k_b_sweep<T, 4>), dim3(b->sweep_grid), dim3(sweep_waves<T>() * kWave), b->sweep_lds, b->stream,
-                       S, st, (const int2*)b->d_items, b->nitems, b->d_next);
-  else
-    hipLaunchKernelGGL((k_b_sweep<T, 2>), dim3(b->sweep_grid), dim3(sweep_waves<T>() * kWave), b->sweep_lds, b->stream,
-                       S, st, (const int2*)b->d_items, b->nitems, b->d_next);
-  hipLaunchKernelGGL(k_b_sum<T>, dim3(n), dim3(256), 0, b->stream, S, n, b->d_step, b->d_res, 1);
+  batch_sweep_launch<T>(b, S, st, 2, 1);
+  hipLaunchKernelGGL(k_b_sum<T>, dim3(n), dim3(256), 0, b->stream, S, n, b->d_step, b->d_res, 1, 0, (unsigned*)nullptr);
   BHIP(b, hipGetLastError());
   return SALMON_OK;
 }

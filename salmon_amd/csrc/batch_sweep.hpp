@@ -729,9 +729,5 @@ __global__ void __launch_bounds__(sweep_waves<T>() * kWave) __attribute__((amdgp
   }
 }
 
-__global__ void k_b_qreset(int* next) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) *next = 0;
-}
-
 }  // namespace batch
 }  // namespace salmon
