@@ -390,10 +390,16 @@ int observe_rows(salmon_ctx* c, const double* kbase, double ax, double ay, doubl
 }
 
 // rho(p) = sum over nchunk partials (nchunk, NL), in a fixed order and with
-// enough threads: slices of <= 16 partials, then the sum of the slices
+// enough threads: more than kDensityChunks of them (the fused step's, one per
+// workgroup) in slices of >= 16 first, then the sum of the slices
 constexpr int kRhoMaxSlices = 64;
 int density_reduce(salmon_ctx* c, const double* part, int nchunk) {
   const int NL = c->g.NL;
+  if (nchunk <= kDensityChunks) {
+    hipLaunchKernelGGL(k_density_final, dim3((NL + 255) / 256), dim3(256), 0, c->stream, part, nchunk, NL, c->d_rho);
+    LAUNCHCHK(c);
+    return SALMON_OK;
+  }
   if (!c->d_rho_part2) {
     int r = dalloc(c, &c->d_rho_part2, (size_t)kRhoMaxSlices * NL);
     if (r) return r;
@@ -414,7 +420,7 @@ int density_dev(salmon_ctx* c) {
   Region reg(c, SALMON_LOG_PSI_RHO);
   const int NL = c->g.NL;
   if (!c->d_rho_part) {
-    c->rho_chunks = std::max(1, std::min(c->NKB, std::max(1, 4096 * 1024 / std::max(1, NL))));
+    c->rho_chunks = std::max(1, std::min({c->NKB, kDensityChunks, std::max(1, 4096 * 1024 / std::max(1, NL))}));
     int r = dalloc(c, &c->d_rho_part, (size_t)c->rho_chunks * NL);
     if (r) return r;
   }

@@ -479,7 +479,12 @@ __global__ void __launch_bounds__(256) k_sum_rows(const double* __restrict__ row
   }
 }
 
-// Density partials: part(c, p) = sum over orbitals of chunk c of occ |psi(p)|^2
+// Density partials: part(c, p) = sum over orbitals of chunk c of occ |psi(p)|^2,
+// at most kDensityChunks of them, which one launch then adds up: a partial per
+// orbital and a stage between cost a launch of 4.5 us on small systems and a
+// write and a read of half the orbitals' size on large ones (240 us for 2048
+// FP64 orbitals of 32^3).
+constexpr int kDensityChunks = 32;
 template <typename T>
 __global__ void __launch_bounds__(256) k_density_part(const cplx<T>* __restrict__ zu, int NKB, int NL, int per_chunk,
                                                       const double* __restrict__ occv, double* __restrict__ part) {
@@ -488,6 +493,7 @@ __global__ void __launch_bounds__(256) k_density_part(const cplx<T>* __restrict_
   if (p >= NL) return;
   const int o0 = c * per_chunk, o1 = min(NKB, o0 + per_chunk);
   double r = 0;
+#pragma unroll 8
   for (int o = o0; o < o1; ++o) {
     const cplx<T> e = zu[(size_t)o * NL + p];
     const double er = e.re, ei = e.im;
