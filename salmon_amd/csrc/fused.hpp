@@ -1220,9 +1220,20 @@ static int fused_step(salmon_ctx* c, const double* amid, const double* aobs, dou
   const int threads = 256 * (sizeof(T) == 8 ? kFusedXS64 : kFusedXS32);
   const int by_regs = std::max(1, (sizeof(T) == 8 ? kFusedWPE64 : kFusedWPE32) * 4 * 64 / threads);
   const int per_cu = std::min(sizeof(T) == 8 ? 1 : 2, by_regs);
-  const int target = 2 * ncu * per_cu;
-  int bpw = (c->NKB + target - 1) / target;
-  bpw = std::max(1, std::min(bpw, c->NB));
+  // orbitals per workgroup (of one k point): the least rounds * (orbitals + set-up)
+  // over the rounds of resident workgroups.  A complex64 orbital takes 20 us and the
+  // set-up (phases, tables into LDS) 19, FP64 45 and about as much: 64 k x 32
+  // complex64 orbitals in one round of 8 each instead of two of 4, 201 -> 188 us.
+  int bpw = 1;
+  long best = -1;
+  for (int b = 1; b <= c->NB; ++b) {
+    const long wgs = (long)c->NK * ((c->NB + b - 1) / b), slots = (long)ncu * per_cu;
+    const long cost = (wgs + slots - 1) / slots * (2 * b + (sizeof(T) == 4 ? 2 : 1));
+    if (best < 0 || cost < best) {
+      best = cost;
+      bpw = b;
+    }
+  }
   const int nbg = (c->NB + bpw - 1) / bpw;
   const int nwg = c->NK * nbg;
   if (nwg > f->nwg_alloc) {
