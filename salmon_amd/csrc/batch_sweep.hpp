@@ -15,9 +15,10 @@
 // come from the current plane, which the team stores in one of two LDS plane
 // buffers (x parity) before a barrier; a column takes col_stride<ZB> slots
 // there, one more than ZB for even ZB, so that the lanes' 8- and 16-byte
-// reads fall in distinct banks.  The per-point operands of plane x+1 (the
+// reads fall in distinct banks.  The per-point operands of a plane (the
 // potential, and for the fold the orbital and its first two H applications)
-// are loaded during step x, before the window load of plane x+5.
+// are loaded at the start of its step (complex64) or of the one before (FP64),
+// before the window load of plane x+5.
 #pragma once
 #include "batch.hpp"
 

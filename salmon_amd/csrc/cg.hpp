@@ -7,8 +7,8 @@
 // iteration (<x|H|x>, |g|^2, the 2x2 Rayleigh-Ritz coefficients, the exit
 // flag) lives in device memory, so a band's whole iteration sequence is
 // enqueued without a host round trip: reductions end in the last-arriving
-// block of each k, which sums the per-block partials in block order (a fixed
-// order, so results do not depend on scheduling) and computes the scalar.
+// block of each k, which sums the per-block partials in a fixed order (so
+// results do not depend on scheduling) and computes the scalar.
 // A k whose band met the exit test (|ev - <x|H|x>| < 1e-15, CG.f90:114)
 // skips the remaining iteration kernels.
 #pragma once

@@ -483,8 +483,11 @@ int gram_schmidt_multi_fwd(salmon_ctx* c, cplx<double>* zu) {
   int r = ensure_work(c);
   if (r || (r = gs_ensure(c))) return r;
   int done = 0;
-  if ((r = gram_schmidt_panels(c, zu, &done)) || done) return r;
-  // nearly dependent (or not finite) bands: band by band
+  // a panel costs four launches and a wait for its flags whatever its bands: 1, 2, 3
+  // and 4 bands of 16^3 at 8 k points take 82, 84, 85 and 85 us in panels, 12, 40, 66
+  // and 92 band by band (8x21x32 at 15 k points 82, 86, 89, 89 and 27, 48, 80, 111)
+  if (c->NB > 3 && ((r = gram_schmidt_panels(c, zu, &done)) || done)) return r;
+  // few, nearly dependent (or not finite) bands: band by band
   GsState* s = (GsState*)c->gs;
   const long key[4] = {(long)(uintptr_t)zu, c->NB, c->NK, 0};
   return graph_run(c, s->g_gs, key, [&]() { return gram_schmidt_multi(c, zu); });
