@@ -9,11 +9,15 @@
 //   P <- (P - Q C) R^-1 = [Q P] W in one more (k_gsb_apply).
 // R is upper triangular with a positive diagonal, so the result is that of the
 // sequential loop (Gram_Schmidt_ompk, ARTED/GS/Gram_Schmidt.f90:41-51) up to
-// rounding: the first round leaves an overlap of eps * cond^2, the second, on
-// nearly orthonormal bands, of eps.  Bands that lose more than a factor 1e-8 of
-// their squared norm to the others (or are not finite) set their k point's flag:
-// its bands stay as they are from there on, and the caller runs the band-by-band
-// form.
+// rounding: the first round leaves an overlap of eps * kappa^2, the second, on
+// nearly orthonormal bands, of eps.  kappa^2 = sum_ij |R^-1(i,j)|^2 |P_i|^2 is the
+// squared condition of the panel, its bands scaled to norm one, against the
+// finished bands: it also sees what no pivot of R shows by itself, bands that each
+// keep a part of their norm but lose it in turn (b_j = e_{j-1} + e_j / 30: every
+// pivot 1e-3, and twelve of them dependent to rounding).  A panel past kGsbCond, or
+// one that is not finite, sets its k point's flag before it changes: the k point's
+// bands stay as they are from there on, and the caller runs the band-by-band form.
+// Up to the limit the results differ from that form's by eps * kappa, 1e-12.
 //
 // Per panel round that is two launches for the finished bands' bytes read twice
 // and the panel's read twice and written once.  Measured, band by band and in
@@ -31,7 +35,7 @@ namespace salmon {
 namespace cg {
 
 constexpr int kPanel = 16;
-constexpr double kGsbPivot = 1e-8;
+constexpr double kGsbCond = 1e8;
 
 struct GsBlock {
   cplx<double>* zu;     // (NK, NB, NL)
@@ -153,20 +157,16 @@ __global__ void __launch_bounds__(256) k_gsb_overlap(GsBlock b, int j0, int np) 
   // the last tile's block: G - C^H C, its Cholesky factor and inverse, W.  C comes
   // in tiles of 16 bands, a value per thread, the next one while one is used.
   __shared__ cplx<double> G[16][17], R[16][17], Ct[16][17];
-  __shared__ int bad;
+  __shared__ double norm[16], cond[4];  // squared norms of the panel's bands before; sums of kappa^2 by wave
   const int row = t / 16, col = t & 15;
   const cplx<double>* C = b.C + (size_t)k * b.NB * 16 + row * 16 + col;
   auto next = [&](int i) { return load_agent(C + (size_t)min(i, j0 - 16) * 16); };  // (j0: whole panels)
-  if (t == 0) bad = 0;
-  double g0 = 0.0;  // the band's squared norm before
   {
     cplx<double> v{row == col ? 1.0 : 0.0, 0.0}, ct{0, 0};
     if (j0 > 0) ct = next(0);
     if (row < np && col < np) {
       v = load_agent(C + (size_t)j0 * 16);
-      if (row == col) g0 = v.re;
-    } else if (row == col) {
-      g0 = 1.0;
+      if (row == col) norm[row] = v.re;
     }
     for (int i0 = 0; i0 < j0; i0 += 16) {
       Ct[row][col] = ct;
@@ -189,8 +189,7 @@ __global__ void __launch_bounds__(256) k_gsb_overlap(GsBlock b, int j0, int np) 
   // right-looking elimination of the upper triangle; R becomes the inverse of the
   // factor: column j of R^-1 follows the same row operations from the right
   for (int j = 0; j < 16; ++j) {
-    const double d = G[j][j].re;
-    if (row == j && col == j && !(d > kGsbPivot * g0)) bad = 1;
+    const double d = G[j][j].re;  // (not positive: infinities or NaN in R)
     const double inv = 1.0 / sqrt(d);
     const cplx<double> u{G[j][col].re * inv, G[j][col].im * inv};  // row j of the factor
     const cplx<double> l{G[j][row].re * inv, G[j][row].im * inv};
@@ -208,7 +207,13 @@ __global__ void __launch_bounds__(256) k_gsb_overlap(GsBlock b, int j0, int np) 
     }
     __syncthreads();
   }
-  if (bad) {
+  {
+    const cplx<double> r = R[row][col];
+    const double q = wave_sum(row < np && col < np ? (r.re * r.re + r.im * r.im) * norm[row] : 0.0);
+    if (lane == 0) cond[wv] = q;
+  }
+  __syncthreads();
+  if (!((cond[0] + cond[1]) + (cond[2] + cond[3]) <= kGsbCond)) {
     if (t == 0) b.flag[k] = 1;
     return;
   }
