@@ -546,22 +546,22 @@ __global__ void __launch_bounds__(256) k_cg_h(State S, const cplx<double>* __res
   const int k = blockIdx.y, c = blockIdx.x;
   const int skip = ROLE == H_RR ? S.done[k] : 0;
   double* sc = S.sc + k * kNS;
-  const int p = c * 256 + threadIdx.x;
+  const int p = c * 256 + threadIdx.x, pc = min(p, S.NL - 1);
   const double s = sc[ROLE == H_EFIN ? XN : SN];
   double sum[3] = {0.0, 0.0, 0.0};
+  const size_t i = (size_t)k * S.NL + pc;
+  const int tp = kb.pt2t[pc];
+  cplx<double> xp{0, 0};
+  if (ROLE == H_RR) xp = x[i];
+  double kx, ky, kz;
+  orbital_k(kac, S.NK, k, 0, 0, 0, kx, ky, kz);
+  cplx<double> e, t;
+  double V;
+  cplx<double> f = stencil_point<double>(v + (size_t)k * S.NL, pc, kx, ky, kz, vloc, g, e, V);
+  loaded(f);
+  loaded(xp);
+  if (ROLE == H_RR && skip) return;  // the whole block, threads past the grid among them: barriers follow
   if (p < S.NL) {
-    const size_t i = (size_t)k * S.NL + p;
-    const int tp = kb.pt2t[p];
-    cplx<double> xp{0, 0};
-    if (ROLE == H_RR) xp = x[i];
-    double kx, ky, kz;
-    orbital_k(kac, S.NK, k, 0, 0, 0, kx, ky, kz);
-    cplx<double> e, t;
-    double V;
-    cplx<double> f = stencil_point<double>(v + (size_t)k * S.NL, p, kx, ky, kz, vloc, g, e, V);
-    loaded(f);
-    loaded(xp);
-    if (ROLE == H_RR && skip) return;  // (of all threads of the block: one k)
     if (tv) t = cplx<double>{f.re - V * e.re, f.im - V * e.im};
     if (tp >= 0) {
       const cplx<double>* d = dps + (size_t)k * kb.NPI;
