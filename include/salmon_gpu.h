@@ -249,14 +249,20 @@ int salmon_gpu_rt_run(salmon_ctx *ctx, const double *ac, int nsteps, double dt, 
  * copied: their resident orbitals advance; they must not be used elsewhere
  * while the batch runs and must outlive it.  All contexts share the batch's
  * precision, A(t) and dt.
- * Two step kernels: SALMON_BATCH_SWEEP, one persistent launch per step whose
+ * Two kinds of step: SALMON_BATCH_SWEEP, one persistent launch per step whose
  * workgroups take (system, orbitals) items from a device work counter and
  * run each orbital's whole step (grids of at least 8 points per axis whose x
  * plane splits into at most 256 columns of up to 4 z points in complex64, 512
  * columns of up to 2 z points in FP64), and SALMON_BATCH_PHASES,
  * one launch per phase over all systems (any grid).  SALMON_BATCH_AUTO (the
- * default) takes the sweep when every system fits it; salmon_gpu_batch_kernel
- * reports the kernel in use after tune (-1 before).  For the phase kernel
+ * default) takes the sweep when every system fits it, and in its place the
+ * resident kernel -- every orbital in the LDS of one workgroup, up to 32 steps
+ * per launch -- when every system fits that too (orbital and sphere points
+ * within 160 KB, up to four projectors per atom) and the batch has at most
+ * four orbitals per compute unit.  salmon_gpu_batch_kernel reports the kind in
+ * use after tune (-1 before; SALMON_BATCH_SWEEP also for the resident kernel),
+ * salmon_gpu_batch_resident whether it is the resident kernel (1, 0; -1 before
+ * tune).  SALMON_BATCH_SWEEP asked for is the sweep itself.  For the phase kernel
  * salmon_gpu_batch_tune times the stencil's z blocking (1, 2, 4 or 8 points
  * per thread along z) per grid shape and keeps the fastest (rt_run tunes on
  * first use); salmon_gpu_batch_zblock reports the choice.  Outputs:
@@ -269,6 +275,7 @@ int salmon_gpu_batch_add(salmon_batch *batch, salmon_ctx *ctx);
 /* SALMON_ERR_ARG from tune/rt_run if SALMON_BATCH_SWEEP is asked for and a system does not fit it */
 int salmon_gpu_batch_set_kernel(salmon_batch *batch, int kernel);
 int salmon_gpu_batch_kernel(const salmon_batch *batch);
+int salmon_gpu_batch_resident(const salmon_batch *batch);
 int salmon_gpu_batch_tune(salmon_batch *batch);
 int salmon_gpu_batch_zblock(salmon_batch *batch, int sys);
 int salmon_gpu_batch_rt_run(salmon_batch *batch, const double *ac, int nsteps, double dt, double *jt, double *et,
@@ -290,19 +297,23 @@ int salmon_gpu_batch_finalize(salmon_batch *batch);
  * per step; ETRS or the self-consistent potential: the Taylor-only
  * launch(es), density and potential, one observables launch per step; the
  * context as a batch of one on its own stream, its work buffers four times
- * the orbitals' size; a set-up that fails falls back); the streamed kernels
+ * the orbitals' size; a set-up that fails falls back), or in its place the
+ * batches' resident kernel where it applies; the streamed kernels
  * otherwise.  SALMON_PATH_STREAMED forces the streamed kernels (and frees
  * the sweep's work buffers),
- * SALMON_PATH_SWEEP the persistent sweep (rt_run then fails with
+ * SALMON_PATH_SWEEP the persistent sweep itself (rt_run then fails with
  * SALMON_ERR_UNSUPPORTED where it does not apply).  Like the reference's
  * build-time stencil selection (ARTED/stencil/CMakeLists.txt:1-52) the choice
  * changes the code path, not the results beyond rounding.  salmon_gpu_path
  * returns the path rt_run takes (SALMON_PATH_FUSED, SALMON_PATH_SWEEP or
- * SALMON_PATH_STREAMED).  The other entry points (hamiltonian, hpsi, the
- * observables) take the streamed kernels. */
+ * SALMON_PATH_STREAMED; SALMON_PATH_SWEEP also where the resident kernel is
+ * taken, which salmon_gpu_resident tells once the path is set up: 1, 0, and -1
+ * before its first use and on the other paths).  hamiltonian and the
+ * observables take the same path, hpsi the streamed kernels. */
 enum { SALMON_PATH_AUTO = 0, SALMON_PATH_STREAMED = 1, SALMON_PATH_FUSED = 2, SALMON_PATH_SWEEP = 3 };
 int salmon_gpu_set_path(salmon_ctx *ctx, int path);
 int salmon_gpu_path(salmon_ctx *ctx);
+int salmon_gpu_resident(salmon_ctx *ctx);
 
 /* Propagator of salmon_gpu_rt_run: the input variable propagator and its
  * dispatch in dt_evolve_KB (ARTED/RT/dt_evolve.f90:28-59).  MIDPOINT: one

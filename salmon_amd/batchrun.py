@@ -47,7 +47,7 @@ def run(nsys=64, steps=10, scale=1.0, precisions=(gpu.FP64, gpu.MIXED), sequenti
             tt = time.time()
             zb = b.tune()
             tune_s = time.time() - tt
-            kern = "sweep" if b.kernel() == gpu.BATCH_SWEEP else "phases"
+            kern = "phases" if b.kernel() == gpu.BATCH_PHASES else "resident" if b.resident() == 1 else "sweep"
             b.rt_run(ac[:2], 1, 0.08)  # warm-up step (captures the graph)
             tt = time.time()
             r = b.rt_run(ac[1:], steps, 0.08)
@@ -62,7 +62,7 @@ def run(nsys=64, steps=10, scale=1.0, precisions=(gpu.FP64, gpu.MIXED), sequenti
         res["algorithmic_bytes_per_step"] = 12 * S * pts
         res["roofline_gbs"] = res["algorithmic_bytes_per_step"] / (res["ms_per_step"] * 1e-3) / 1e9
         res["roofline_frac"] = res["roofline_gbs"] / HBM_PEAK_GBS
-        zdesc = f"z blocking {res['zblock']}" if kern == "phases" else "persistent sweep"
+        zdesc = {"phases": f"z blocking {res['zblock']}", "sweep": "persistent sweep", "resident": "resident kernel"}[kern]
         log(f"[batch] {name}: {res['ms_per_step']:.2f} ms/step, {res['orbital_steps_per_s']:.3e} orbital-steps/s "
             f"(tune {tune_s:.1f} s, {zdesc}); {res['roofline_gbs']:.0f} GB/s of algorithmic "
             f"bytes = {res['roofline_frac']:.3f} of {HBM_PEAK_GBS:.0f} GB/s")

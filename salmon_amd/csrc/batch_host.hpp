@@ -47,6 +47,7 @@ struct salmon_batch {
   std::vector<ResClass> res;
   const ResTab* d_restab = nullptr;
   bool resident = false;
+  bool resident_ok = true;        // not asked for the sweep itself
   unsigned sweep_grid = 0;
   size_t sweep_lds = 0;
   // one Taylor step at caller-given k points (batch_taylor): descriptors whose
@@ -381,7 +382,7 @@ static int batch_build(salmon_batch* b) {
   const int n = (int)b->ctx.size();
   std::vector<Sys<T>> S(n);
   b->max_ph = 0;
-  bool sweeps = b->kernel_req != SALMON_BATCH_PHASES;
+  bool sweeps = b->kernel_req != SALMON_BATCH_PHASES && b->resident_ok;
   for (int i = 0; i < n; ++i) {
     salmon_ctx* c = b->ctx[i];
     Sys<T>& y = S[i];

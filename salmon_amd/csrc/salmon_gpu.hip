@@ -742,10 +742,12 @@ int solo_prepare(salmon_ctx* c) {
     c->solo_gen = c->gen;
   }
   salmon_batch* b = c->solo;
-  if (c->solo_gen != c->gen) {
+  const bool resident_ok = c->path != SALMON_PATH_SWEEP;
+  if (c->solo_gen != c->gen || b->resident_ok != resident_ok) {
     (void)hipStreamSynchronize(c->stream);
     batch_release(b);
     b->tuned = false;
+    b->resident_ok = resident_ok;
     c->solo_gen = c->gen;
     c->solo_fail = false;
   }
@@ -1868,12 +1870,18 @@ int salmon_gpu_batch_set_kernel(salmon_batch* b, int kernel) {
   batch_release(b);
   b->tuned = false;
   b->kernel_req = kernel;
+  b->resident_ok = kernel == SALMON_BATCH_AUTO;
   return SALMON_OK;
 }
 
 int salmon_gpu_batch_kernel(const salmon_batch* b) {
   if (!b || !b->ready || !b->tuned) return -1;
   return b->sweep ? SALMON_BATCH_SWEEP : SALMON_BATCH_PHASES;
+}
+
+int salmon_gpu_batch_resident(const salmon_batch* b) {
+  if (!b || !b->ready || !b->tuned) return -1;
+  return b->resident ? 1 : 0;
 }
 
 int salmon_gpu_batch_tune(salmon_batch* b) {
@@ -1980,6 +1988,13 @@ int salmon_gpu_set_path(salmon_ctx* c, int path) {
 int salmon_gpu_path(salmon_ctx* c) {
   if (!c) return -1;
   return rt_path(c);
+}
+
+int salmon_gpu_resident(salmon_ctx* c) {
+  if (!c || rt_path(c) != SALMON_PATH_SWEEP || !c->solo || c->solo_gen != c->gen ||
+      c->solo->resident_ok != (c->path != SALMON_PATH_SWEEP))
+    return -1;
+  return salmon_gpu_batch_resident(c->solo);
 }
 
 void* salmon_gpu_stream(salmon_ctx* c) { return c ? (void*)c->stream : nullptr; }

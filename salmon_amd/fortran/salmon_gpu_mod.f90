@@ -304,6 +304,11 @@ module salmon_gpu
       type(c_ptr), value :: batch
     end function
 
+    integer(c_int) function salmon_gpu_batch_resident(batch) bind(C, name="salmon_gpu_batch_resident")
+      import :: c_int, c_ptr
+      type(c_ptr), value :: batch
+    end function
+
     integer(c_int) function salmon_gpu_batch_tune(batch) bind(C, name="salmon_gpu_batch_tune")
       import :: c_int, c_ptr
       type(c_ptr), value :: batch
@@ -353,6 +358,11 @@ module salmon_gpu
     end function
 
     integer(c_int) function salmon_gpu_path(ctx) bind(C, name="salmon_gpu_path")
+      import :: c_int, c_ptr
+      type(c_ptr), value :: ctx
+    end function
+
+    integer(c_int) function salmon_gpu_resident(ctx) bind(C, name="salmon_gpu_resident")
       import :: c_int, c_ptr
       type(c_ptr), value :: ctx
     end function

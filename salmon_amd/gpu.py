@@ -102,6 +102,7 @@ SIGNATURES = {
     "salmon_gpu_batch_add": [_vp, _vp],
     "salmon_gpu_batch_set_kernel": [_vp, _ci],
     "salmon_gpu_batch_kernel": [_vp],
+    "salmon_gpu_batch_resident": [_vp],
     "salmon_gpu_batch_tune": [_vp],
     "salmon_gpu_batch_zblock": [_vp, _ci],
     "salmon_gpu_batch_rt_run": [_vp, _vp, _ci, _cd, _vp, _vp, _vp],
@@ -110,6 +111,7 @@ SIGNATURES = {
     "salmon_gpu_batch_finalize": [_vp],
     "salmon_gpu_set_path": [_vp, _ci],
     "salmon_gpu_path": [_vp],
+    "salmon_gpu_resident": [_vp],
     "salmon_gpu_synchronize": [_vp],
     "salmon_gpu_timer_enable": [_vp, _ci],
     "salmon_gpu_timer_reset": [_vp],
@@ -391,6 +393,10 @@ class Context:
     def path(self):
         return lib().salmon_gpu_path(self._h)
 
+    def resident(self):
+        """1 if the LDS-resident kernel runs in place of the sweep (PATH_AUTO), 0 if not; -1 before its first use."""
+        return lib().salmon_gpu_resident(self._h)
+
     def synchronize(self):
         self._check(lib().salmon_gpu_synchronize(self._h), "synchronize")
 
@@ -500,8 +506,13 @@ class Batch:
         self._check(lib().salmon_gpu_batch_set_kernel(self._h, int(kernel)), "batch_set_kernel")
 
     def kernel(self):
-        """The step kernel in use (BATCH_PHASES or BATCH_SWEEP); -1 before tune."""
+        """The kind of step in use (BATCH_PHASES or BATCH_SWEEP, which the resident
+        kernel counts as); -1 before tune."""
         return lib().salmon_gpu_batch_kernel(self._h)
+
+    def resident(self):
+        """1 if the LDS-resident kernel runs the steps (BATCH_AUTO only), 0 if not; -1 before tune."""
+        return lib().salmon_gpu_batch_resident(self._h)
 
     def tune(self):
         self._check(lib().salmon_gpu_batch_tune(self._h), "batch_tune")
