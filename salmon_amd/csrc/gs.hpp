@@ -85,6 +85,8 @@ static void gs_free(salmon_ctx* c) {
   GsState* s = (GsState*)c->gs;
   if (!s) return;
   for (void* p : s->bufs) (void)hipFree(p);
+  (void)hipFree(s->ph);
+  (void)hipFree(s->dps);
   for (void* p : s->smp_bufs) (void)hipFree(p);
   for (void* p : s->inf.bufs) (void)hipFree(p);
   graph_free(s->g_cg);
@@ -121,9 +123,26 @@ static void kinetic_tables(const Grid& g, std::vector<double>& tw, std::vector<d
   }
 }
 
+// The tables of the sphere points, whose number changes when an atom moves; the
+// rest of the state, recorded samples and targets among it, does not depend on them.
+static int gs_ensure_points(salmon_ctx* c, GsState* s) {
+  if (s->ph && s->NPI == c->kb.NPI) return SALMON_OK;
+  (void)hipFree(s->ph);
+  (void)hipFree(s->dps);
+  s->ph = s->dps = nullptr;
+  s->NPI = c->kb.NPI;
+  const size_t bytes = sizeof(cplx<double>) * std::max<size_t>(1, (size_t)s->NK * s->NPI);
+  if (hipMalloc((void**)&s->dps, bytes) != hipSuccess || hipMalloc((void**)&s->ph, bytes) != hipSuccess) {
+    (void)hipFree(s->dps);
+    s->ph = s->dps = nullptr;
+    return fail(c, SALMON_ERR_NOMEM, "ground-state sphere points (%zu bytes)", bytes);
+  }
+  return SALMON_OK;
+}
+
 static int gs_ensure(salmon_ctx* c) {
   GsState* s = (GsState*)c->gs;
-  if (s && s->NK == c->NK && s->NB == c->NB && s->Nlma == c->kb.Nlma && s->NPI == c->kb.NPI) return SALMON_OK;
+  if (s && s->NK == c->NK && s->NB == c->NB && s->Nlma == c->kb.Nlma) return gs_ensure_points(c, s);
   gs_free(c);
   s = new GsState();
   c->gs = s;
@@ -131,7 +150,6 @@ static int gs_ensure(salmon_ctx* c) {
   s->NB = c->NB;
   s->NL = c->g.NL;
   s->Nlma = c->kb.Nlma;
-  s->NPI = c->kb.NPI;
   s->nchunk = (s->NL + kChunk - 1) / kChunk;
   s->ngroup = (s->NB + kJG - 1) / kJG;
   s->pstride = std::max(s->nchunk * s->ngroup * kPartQ, (s->NL + kSubPts - 1) / kSubPts * 5);
@@ -139,8 +157,7 @@ static int gs_ensure(salmon_ctx* c) {
   int r;
   for (int i = 0; i < 10; ++i)
     if ((r = gs_alloc(c, s, &s->w[i], nv))) return r;
-  if ((r = gs_alloc(c, s, &s->ph, (size_t)s->NK * s->NPI))) return r;
-  if ((r = gs_alloc(c, s, &s->dps, (size_t)s->NK * s->NPI))) return r;
+  if ((r = gs_ensure_points(c, s))) return r;
   if ((r = gs_alloc(c, s, &s->sc, (size_t)s->NK * kNS))) return r;
   if ((r = gs_alloc(c, s, &s->done, (size_t)s->NK))) return r;
   if ((r = gs_alloc(c, s, &s->iters, (size_t)s->NK * s->NB))) return r;
