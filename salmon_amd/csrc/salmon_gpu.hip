@@ -420,7 +420,9 @@ int density_dev(salmon_ctx* c) {
   Region reg(c, SALMON_LOG_PSI_RHO);
   const int NL = c->g.NL;
   if (!c->d_rho_part) {
-    c->rho_chunks = std::max(1, std::min({c->NKB, kDensityChunks, std::max(1, 4096 * 1024 / std::max(1, NL))}));
+    const bool few = kDensityChunks * ((NL + 255) / 256) * (int)sizeof(cplx<T>) < kDensityFewBytes;
+    const int most = few ? std::max(kDensityChunks, c->NKB / kDensityOrbitals) : kDensityChunks;
+    c->rho_chunks = std::max(1, std::min({c->NKB, most, std::max(1, 4096 * 1024 / std::max(1, NL))}));
     int r = dalloc(c, &c->d_rho_part, (size_t)c->rho_chunks * NL);
     if (r) return r;
   }

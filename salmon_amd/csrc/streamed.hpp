@@ -480,11 +480,18 @@ __global__ void __launch_bounds__(256) k_sum_rows(const double* __restrict__ row
 }
 
 // Density partials: part(c, p) = sum over orbitals of chunk c of occ |psi(p)|^2,
-// at most kDensityChunks of them, which one launch then adds up: a partial per
+// kDensityChunks of them at most, which one launch then adds up: a partial per
 // orbital and a stage between cost a launch of 4.5 us on small systems and a
 // write and a read of half the orbitals' size on large ones (240 us for 2048
-// FP64 orbitals of 32^3).
+// FP64 orbitals of 32^3).  Where the blocks of 32 are too few to have the
+// memory busy (160 with FP64 values, 320 with complex64), one partial per
+// kDensityOrbitals orbitals if that is more of them: 8^3 x 16384 / 32768 / 65536
+// complex64 orbitals took 54 / 82 / 143 us in 32, 43 / 46 / 66 so, 12^3 x 32768 123
+// and 109; above the line 32 are faster (12^3 x 32768 FP64 168 and 181, 12x14x16 x
+// 32768 and 16^3 x 16384 complex64 150 and 159, 112 and 130).
 constexpr int kDensityChunks = 32;
+constexpr int kDensityOrbitals = 256;
+constexpr int kDensityFewBytes = 160 * 16;  // blocks times the size of a value
 template <typename T>
 __global__ void __launch_bounds__(256) k_density_part(const cplx<T>* __restrict__ zu, int NKB, int NL, int per_chunk,
                                                       const double* __restrict__ occv, double* __restrict__ part) {
