@@ -126,14 +126,80 @@ static std::array<int, 2> sweep_shape(const Grid& g) {
 // The resident kernel's plan: taken where it covers every system of the batch
 // (a grid of its shapes whose orbital, with the sphere points' tables, fits in
 // LDS, up to kResLpa projectors per atom, images within two cells) and the
-// orbitals are at most kResRounds per compute unit.  It runs one workgroup per
-// compute unit, so its time is about 10 (8^3) to 60 (16^3) us a step times the
-// rounds; the sweep's is nearly flat up to there (70 to 330 us for up to 256
-// orbitals) and then grows more slowly.  Beside systems that need the sweep the
-// sweep takes all: its work queue fills the chip across systems.  Builds the
-// tables, work lists and rows; b->resident stays false if the plan does not apply.
+// orbitals are at most kResRounds per compute unit) and is not expected to be
+// slower than the sweep by more than its fewer launches give back (resident_pays).
+// Beside systems that need the sweep the sweep takes all: its work queue fills the
+// chip across systems.  Builds the tables, work lists and rows; b->resident stays
+// false if the plan does not apply.
 constexpr int kResSteps = 32;  // steps per launch (rows kept per orbital)
 constexpr long kResRounds = 4;
+constexpr size_t kSweepMaxLds = 65536;
+
+// LDS of the sweep for one system of the given column length and team size
+template <typename T>
+static size_t sweep_lds_bytes(const Sys<T>& y, const std::array<int, 2>& sh) {
+  const int teams = sweep_waves<T>() / sh[1];
+  const int zb = sh[0], cs = zb % 2 == 0 ? zb + 1 : zb;  // col_stride<zb>()
+  const size_t PS = ((size_t)y.g.NLy * y.g.NLz / zb + 1) * cs;  // plane_slots<zb>(P)
+  return (size_t)kSweepHead + (size_t)teams * (2 * PS + y.kb.Nlma) * sizeof(cplx<T>);
+}
+
+// Time of one H application of all orbitals in the resident kernel against the
+// sweep's.  The resident kernel runs one workgroup per compute unit, so its time is
+// its orbitals' times the rounds; the sweep's is a chain of planes that 4 to 8
+// orbitals per compute unit run at nearly the time of one.  Fits (us) to 380
+// measured pairs (21 grids of 8x8x8 to 18x16x16, 512 to 1024 orbitals, 1 and 6 atoms,
+// both precisions), each within 16 % and 4 to 5 % on average: the resident kernel by
+// its x points per thread and atoms per wave, the sweep by planes, column length,
+// team size and passes over the sphere points, and by how full the chip is.  The
+// lines, 1.1 and in complex64 1.25, are where runs of ten steps (which the resident
+// kernel needs fewer launches for) took as long either way.  Without the comparison 14^3 x 1024 orbitals took 194 us a hamiltonian call
+// in FP64 where the sweep takes 144, 31x8x9 x 1024 193 and 138; 12^3 x 1024 104
+// and 119.
+template <typename T>
+static bool resident_pays(const salmon_batch* b, const std::vector<Sys<T>>& S, int ncu) {
+  constexpr bool f64 = sizeof(T) == 8;
+  const double base[7] = {0, f64 ? 2.2 : 2.0, f64 ? 2.9 : 2.6, f64 ? 4.6 : 3.6, f64 ? 6.6 : 4.5, 0, f64 ? 10.8 : 5.9};
+  struct Class {
+    int px, waves;
+    long n;
+    double t;
+  };
+  std::vector<Class> cls;  // a launch each
+  long items = 0;
+  for (const auto& y : S) {
+    const auto sh = sweep_shape<T>(y.g);
+    if (sweep_lds_bytes(y, sh) > kSweepMaxLds) return true;  // there is no sweep
+    items += (y.NKB + sweep_waves<T>() / sh[1] - 1) / (sweep_waves<T>() / sh[1]);
+    const int px = res_px(y.g), waves = res_waves(y.g, px);
+    const double t = base[px] + (f64 ? 2.6 : 2.2) * y.kb.NI / waves;
+    size_t c = 0;
+    while (c < cls.size() && (cls[c].px != px || cls[c].waves != waves)) ++c;
+    if (c == cls.size()) cls.push_back({px, waves, 0, 0.0});
+    cls[c].n += y.NKB;
+    cls[c].t = std::max(cls[c].t, t);
+  }
+  double res = 0;
+  for (const auto& c : cls) res += c.t * ((c.n + ncu - 1) / ncu);
+  // the sweep: eight waves per compute unit
+  const long slots = (long)ncu * 8 / sweep_waves<T>(), full = items / slots, rest = items % slots;
+  double mean = 0, most = 0;  // an item on a full chip; the longest in the last round
+  for (size_t i = 0; i < S.size(); ++i) {
+    const auto sh = sweep_shape<T>(S[i].g);
+    const std::vector<int>& start = b->ctx[i]->kb_host.start;
+    long passes = 0;
+    for (int a = 0; a < S[i].kb.NI; ++a) passes += (start[a + 1] - start[a] + kWave * sh[1] - 1) / (kWave * sh[1]);
+    const double team = std::log2((double)sh[1]);
+    const double chain = f64 ? (S[i].g.NLx + 2) * (0.62 * sh[0] + 0.1 * team)
+                             : (S[i].g.NLx + 4) * (0.12 + 0.23 * sh[0] + 0.06 * team);
+    const double kb = f64 ? 2.4 * passes - 2.0 : 2.3 * passes - 2.5;
+    const int teams = sweep_waves<T>() / sh[1];
+    mean += (chain * (f64 ? 1.45 : 1.64) + kb) * ((S[i].NKB + teams - 1) / teams) / items;
+    most = std::max(most, chain * (1.0 + (f64 ? 0.45 : 0.64) * rest / slots) + kb);
+  }
+  return res <= (f64 ? 1.1 : 1.25) * (full * mean + (rest ? most : 0.0));
+}
+
 template <typename T>
 static int resident_plan(salmon_batch* b, std::vector<Sys<T>>& S) {
   int dev = 0, ncu = 0;
@@ -147,7 +213,7 @@ static int resident_plan(salmon_batch* b, std::vector<Sys<T>>& S) {
         std::max({g.NLx, g.NLy, g.NLz}) > 200)
       return SALMON_OK;
   }
-  if (orbitals > kResRounds * ncu) return SALMON_OK;
+  if (orbitals > kResRounds * ncu || !resident_pays<T>(b, S, ncu)) return SALMON_OK;
   // all tables and work lists in one device block: offsets first, pointers after its allocation
   std::vector<unsigned char> blob;
   auto put = [&](const void* src, size_t bytes) {
@@ -300,9 +366,7 @@ static int sweep_plan(salmon_batch* b, std::vector<Sys<T>>& S) {
     S[i].sw_zb = sh[0];
     S[i].sw_tw = sh[1];
     const int teams = sweep_waves<T>() / sh[1];
-    const int zb = sh[0], cs = zb % 2 == 0 ? zb + 1 : zb;  // col_stride<zb>()
-    const size_t PS = ((size_t)S[i].g.NLy * S[i].g.NLz / zb + 1) * cs;  // plane_slots<zb>(P)
-    lds = std::max(lds, (size_t)kSweepHead + (size_t)teams * (2 * PS + S[i].kb.Nlma) * sizeof(cplx<T>));
+    lds = std::max(lds, sweep_lds_bytes(S[i], sh));
     for (int o = 0; o < S[i].NKB; o += teams)
       items.push_back({(long)S[i].g.NL * std::min(teams, S[i].NKB - o), (long)i, (long)o});
   }
@@ -344,7 +408,7 @@ static int sweep_plan(salmon_batch* b, std::vector<Sys<T>>& S) {
     S[i].kb_cstart = d + kb.NI;
     S[i].ncolor = nc;
   }
-  if (lds > 65536 || items.empty()) {
+  if (lds > kSweepMaxLds || items.empty()) {
     if (must) return bfail(b, SALMON_ERR_ARG, "the persistent sweep needs %zu bytes of LDS", lds);
     return SALMON_OK;
   }
