@@ -707,11 +707,11 @@ constexpr int kDftMax = 64;
 
 // Grid (blocks of z lines, NLx, NK).
 __global__ void __launch_bounds__(256) k_kin_zy(State S, const cplx<double>* __restrict__ in, cplx<double>* __restrict__ out,
-                                                Grid g, const double* __restrict__ tw) {
+                                                Grid g, int nl, const double* __restrict__ tw) {
   const int k = blockIdx.z;
   if (S.done[k]) return;
   const size_t o = (size_t)k * g.NL + (size_t)blockIdx.y * g.NLy * g.NLz;
-  dft::plane<true>(g.NLz, g.NLy, tw + 4 * kDftMax, tw + 2 * kDftMax, -1.0,
+  dft::plane<true>(g.NLz, g.NLy, nl, tw + 4 * kDftMax, tw + 2 * kDftMax, -1.0,
                    [&](int z, int y) { return in[o + y * g.NLz + z]; },
                    [&](int z, int y, cplx<double> v) { out[o + y * g.NLz + z] = v; });
 }
@@ -732,11 +732,11 @@ __global__ void __launch_bounds__(256) k_kin_x(State S, cplx<double>* __restrict
 
 // Grid (blocks of y lines, NLx, NK).
 __global__ void __launch_bounds__(256) k_kin_yz(State S, const cplx<double>* __restrict__ in, cplx<double>* __restrict__ out,
-                                                Grid g, const double* __restrict__ tw) {
+                                                Grid g, int nl, const double* __restrict__ tw) {
   const int k = blockIdx.z;
   if (S.done[k]) return;
   const size_t o = (size_t)k * g.NL + (size_t)blockIdx.y * g.NLy * g.NLz;
-  dft::plane<false>(g.NLy, g.NLz, tw + 2 * kDftMax, tw + 4 * kDftMax, 1.0,
+  dft::plane<false>(g.NLy, g.NLz, nl, tw + 2 * kDftMax, tw + 4 * kDftMax, 1.0,
                     [&](int y, int z) { return in[o + y * g.NLz + z]; },
                     [&](int y, int z, cplx<double> v) { out[o + y * g.NLz + z] = v; });
 }

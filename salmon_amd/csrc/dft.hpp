@@ -11,46 +11,60 @@
 // blocks without repeating work: the first of its two transforms is formed only
 // for the second axis' lines that the block transforms next.
 #pragma once
+#include <algorithm>
+
 #include "common.hpp"
 
 namespace salmon {
 namespace dft {
 
 constexpr int kTile = 1024;  // grid values staged at a time
-constexpr int kLines = 8;    // least lines of a block's second transform (256 threads; more on short axes)
+constexpr int kLines = 8;    // lines of a block's second transform (256 threads; more on short axes)
+constexpr int kBlocks = 512;
 
-inline __host__ __device__ int plane_lines(int n) { return max(kLines, 256 / n); }  // n: their length
-// dynamic LDS of the plane kernels (first, second: lengths of the first and the second transform's axis)
-inline size_t plane_lds(int first, int second) {
-  return 16 * ((size_t)max(kTile, first) + (size_t)plane_lines(second) * second + first + second);
+// Lines per block of a plane launch for axes of the given lengths: a value per
+// thread, and up to kLines where that leaves two blocks per compute unit.  Few
+// planes of long lines have too few blocks otherwise: eight planes of 8x256 took 183
+// us for the whole solve with kLines, 101 so (a pass per axis 141); 256 and 1024 for
+// kBlocks took 1.18 and 1.33 ms on ten planes of 200x200, 512 1.05.
+inline int plane_lines(int first, int second, long planes) {
+  int nl = std::max(1, 256 / second);
+  while (nl < kLines && planes * ((first + nl) / (nl + 1)) >= kBlocks) ++nl;
+  return nl;
+}
+// dynamic LDS of the plane kernels with nl lines
+inline size_t plane_lds(int first, int second, int nl) {
+  return 16 * ((size_t)std::max(kTile, first) + (size_t)nl * second + first + second);
 }
 
-// sum_m a(m) e^{sgn 2 pi i e m / n}, a(m) at a[m * as]
-__device__ __forceinline__ cplx<double> line_sum(const cplx<double>* a, int as, int n, int e, const double2* w, double sgn) {
+// sum over m = m0, m0 + dm, ... of a(m) e^{sgn 2 pi i e m / n}, a(m) at a[m * as]
+__device__ __forceinline__ cplx<double> line_sum(const cplx<double>* a, int as, int n, int e, const double2* w, double sgn,
+                                                 int m0 = 0, int dm = 1) {
   double re = 0.0, im = 0.0;
-  int j = 0;
+  int j = m0 == 0 ? 0 : e * m0 % n;
+  const int dj = dm == 1 ? e : e * dm % n;
 #pragma unroll 4
-  for (int m = 0; m < n; ++m) {
+  for (int m = m0; m < n; m += dm) {
     const double c = w[j].x, s = sgn * w[j].y;
     const cplx<double> v = a[m * as];
     re += c * v.re - s * v.im;
     im += c * v.im + s * v.re;
-    j += e;
+    j += dj;
     if (j >= n) j -= n;
   }
   return {re, im};
 }
 
-// Both transforms of a plane for kLines or more lines of the second axis.  The
+// Both transforms of a plane for nl lines of the second axis.  The
 // plane's value at (first axis a, second axis b) comes from in(a, b), tiles of
 // whole first-axis lines at a time; out(a, b, value) gets the results of the
-// block's lines a = blockIdx.x * plane_lines(NB) ...  FAST: the first axis is
+// block's nl lines a = blockIdx.x * nl ...  FAST: the first axis is
 // the one of consecutive grid points.
 template <bool FAST, typename IN, typename OUT>
-__device__ __forceinline__ void plane(int NA, int NB, const double* twa, const double* twb, double sgn, IN in, OUT out) {
+__device__ __forceinline__ void plane(int NA, int NB, int nl, const double* twa, const double* twb, double sgn, IN in, OUT out) {
   extern __shared__ __align__(16) unsigned char dft_lds[];
   cplx<double>* tile = (cplx<double>*)dft_lds;
-  const int nl = plane_lines(NB), a0 = blockIdx.x * nl, na = min(nl, NA - a0), t = threadIdx.x;
+  const int a0 = blockIdx.x * nl, na = min(nl, NA - a0), t = threadIdx.x;
   cplx<double>* mid = tile + max(kTile, NA);  // (b, a): first transform's results
   double2* wa = (double2*)(mid + nl * NB);
   double2* wb = wa + NA;
@@ -65,9 +79,18 @@ __device__ __forceinline__ void plane(int NA, int NB, const double* twa, const d
       tile[b * NA + a] = in(a, b0 + b);
     }
     __syncthreads();
-    for (int i = t; i < nb * na; i += 256) {
-      const int b = i / na, a = i - b * na;
-      mid[(b0 + b) * na + a] = line_sum(tile + b * NA, 1, NA, a0 + a, wa, sgn);
+    // long lines leave few sums a tile: neighbouring lanes share each (ten planes of
+    // 200x200 1.47 -> 1.05 ms)
+    int parts = 1;
+    while (parts < 8 && 2 * parts * nb * na <= 256) parts *= 2;
+    for (int i = t; i < nb * na * parts; i += 256) {
+      const int o = i / parts, b = o / na, a = o - b * na;
+      cplx<double> v = line_sum(tile + b * NA, 1, NA, a0 + a, wa, sgn, i - o * parts, parts);
+      for (int s = 1; s < parts; s *= 2) {
+        v.re += __shfl_xor(v.re, s);
+        v.im += __shfl_xor(v.im, s);
+      }
+      if (i == o * parts) mid[(b0 + b) * na + a] = v;
     }
   }
   __syncthreads();

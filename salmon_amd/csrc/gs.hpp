@@ -227,13 +227,14 @@ static State gs_view(salmon_ctx* c, GsState* s) {
 static int kinetic_apply(salmon_ctx* c, GsState* s, const State& S, const cplx<double>* g, cplx<double>* out) {
   namespace dft = salmon::dft;
   const Grid& G = c->g;
-  const int nz = dft::plane_lines(G.NLy), ny = dft::plane_lines(G.NLz);
-  hipLaunchKernelGGL(k_kin_zy, dim3((G.NLz + nz - 1) / nz, G.NLx, s->NK), dim3(256), dft::plane_lds(G.NLz, G.NLy), c->stream, S,
-                     g, s->w[W_T1], G, (const double*)s->tw);
+  const long planes = (long)G.NLx * s->NK;
+  const int nz = dft::plane_lines(G.NLz, G.NLy, planes), ny = dft::plane_lines(G.NLy, G.NLz, planes);
+  hipLaunchKernelGGL(k_kin_zy, dim3((G.NLz + nz - 1) / nz, G.NLx, s->NK), dim3(256), dft::plane_lds(G.NLz, G.NLy, nz), c->stream, S,
+                     g, s->w[W_T1], G, nz, (const double*)s->tw);
   hipLaunchKernelGGL(k_kin_x, dim3(dft::lines_x_blocks(G), s->NK), dim3(256), 0, c->stream, S, s->w[W_T1], G,
                      (const double*)s->tw, (const double*)s->symb);
-  hipLaunchKernelGGL(k_kin_yz, dim3((G.NLy + ny - 1) / ny, G.NLx, s->NK), dim3(256), dft::plane_lds(G.NLy, G.NLz), c->stream, S,
-                     (const cplx<double>*)s->w[W_T1], out, G, (const double*)s->tw);
+  hipLaunchKernelGGL(k_kin_yz, dim3((G.NLy + ny - 1) / ny, G.NLx, s->NK), dim3(256), dft::plane_lds(G.NLy, G.NLz, ny), c->stream, S,
+                     (const cplx<double>*)s->w[W_T1], out, G, ny, (const double*)s->tw);
   LAUNCHCHK(c);
   return SALMON_OK;
 }

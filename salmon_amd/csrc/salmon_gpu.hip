@@ -519,13 +519,13 @@ int scf_potential_on(salmon_ctx* c, const double* rho, bool set_v, int xc, doubl
   namespace dft = salmon::dft;
   const Grid& g = c->g;
   const dim3 bl(256);
-  const int nz = dft::plane_lines(g.NLy), ny = dft::plane_lines(g.NLz);
-  hipLaunchKernelGGL(salmon::scf::k_rho_zy, dim3((g.NLz + nz - 1) / nz, g.NLx), bl, dft::plane_lds(g.NLz, g.NLy), c->stream,
-                     rho, A, g, tw);
+  const int nz = dft::plane_lines(g.NLz, g.NLy, g.NLx), ny = dft::plane_lines(g.NLy, g.NLz, g.NLx);
+  hipLaunchKernelGGL(salmon::scf::k_rho_zy, dim3((g.NLz + nz - 1) / nz, g.NLx), bl, dft::plane_lds(g.NLz, g.NLy, nz), c->stream,
+                     rho, A, g, nz, tw);
   hipLaunchKernelGGL(salmon::scf::k_coulomb_x, dim3(dft::lines_x_blocks(g)), bl, 0, c->stream, A, g, tw);
   // parts only: Vpsl = 0 into a scratch potential (the second grid)
-  hipLaunchKernelGGL(salmon::scf::k_vloc_yz, dim3((g.NLy + ny - 1) / ny, g.NLx), bl, dft::plane_lds(g.NLy, g.NLz), c->stream,
-                     (const cplx<double>*)A, g, tw, rho, set_v ? (const double*)c->d_vpsl : (const double*)nullptr, xc,
+  hipLaunchKernelGGL(salmon::scf::k_vloc_yz, dim3((g.NLy + ny - 1) / ny, g.NLx), bl, dft::plane_lds(g.NLy, g.NLz, ny), c->stream,
+                     (const cplx<double>*)A, g, ny, tw, rho, set_v ? (const double*)c->d_vpsl : (const double*)nullptr, xc,
                      set_v ? c->d_vloc : (double*)B, set_v ? c->d_vloc_f : (float*)nullptr, vh, vxc);
   LAUNCHCHK(c);
   return SALMON_OK;

@@ -16,9 +16,9 @@ constexpr int kMaxN = 256;  // points per axis of the DFT passes (twiddle table 
 
 // rho(x; y, z) to its z and y transforms.  Grid (blocks of z lines, NLx).
 __global__ void __launch_bounds__(256) k_rho_zy(const double* __restrict__ rho, cplx<double>* __restrict__ f, Grid g,
-                                                const double* __restrict__ tw) {
+                                                int nl, const double* __restrict__ tw) {
   const size_t o = (size_t)blockIdx.y * g.NLy * g.NLz;
-  dft::plane<true>(g.NLz, g.NLy, tw + 4 * kMaxN, tw + 2 * kMaxN, -1.0,
+  dft::plane<true>(g.NLz, g.NLy, nl, tw + 4 * kMaxN, tw + 2 * kMaxN, -1.0,
                    [&](int z, int y) { return cplx<double>{rho[o + y * g.NLz + z], 0.0}; },
                    [&](int z, int y, cplx<double> v) { f[o + y * g.NLz + z] = v; });
 }
@@ -60,12 +60,12 @@ __device__ __forceinline__ double pz_vxc(double rho) {
 // V_H from its x-back-transformed rows by the y and z transforms, and Vloc = V_H +
 // Vpsl + V_xc into the FP64 potential and its FP32 copy; vh/vxc (nullable) get the
 // parts.  Grid (blocks of y lines, NLx).
-__global__ void __launch_bounds__(256) k_vloc_yz(const cplx<double>* __restrict__ f, Grid g, const double* __restrict__ tw,
+__global__ void __launch_bounds__(256) k_vloc_yz(const cplx<double>* __restrict__ f, Grid g, int nl, const double* __restrict__ tw,
                                                  const double* __restrict__ rho, const double* __restrict__ vpsl, int xc,
                                                  double* __restrict__ v64, float* __restrict__ v32,
                                                  double* __restrict__ vh, double* __restrict__ vxc) {
   const size_t o = (size_t)blockIdx.y * g.NLy * g.NLz;
-  dft::plane<false>(g.NLy, g.NLz, tw + 2 * kMaxN, tw + 4 * kMaxN, 1.0,
+  dft::plane<false>(g.NLy, g.NLz, nl, tw + 2 * kMaxN, tw + 4 * kMaxN, 1.0,
                     [&](int y, int z) { return f[o + y * g.NLz + z]; },
                     [&](int y, int z, cplx<double> r) {
                       const size_t p = o + y * g.NLz + z;
