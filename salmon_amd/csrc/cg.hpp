@@ -829,9 +829,12 @@ __global__ void __launch_bounds__(256) k_rotate_bands(const cplx<double>* __rest
 
 // Gram-Schmidt step of band ib in place (Gram_Schmidt_ompk,
 // ARTED/GS/Gram_Schmidt.f90:43-50): v -= sum_{j<ib} zs_j B_j; with_norm ends
-// with SN = 1/sqrt(|v|^2 Hxyz).  Grid (nvec, NK).
-__global__ void __launch_bounds__(256) k_gs_sub(State S, cplx<double>* __restrict__ zu, int ib, int with_norm) {
+// with SN = 1/sqrt(|v|^2 Hxyz).  check_done: not of k points whose done flag is set.
+// Grid (nvec, NK).
+__global__ void __launch_bounds__(256) k_gs_sub(State S, cplx<double>* __restrict__ zu, int ib, int with_norm,
+                                                int check_done) {
   const int k = blockIdx.y, c = blockIdx.x;
+  if (check_done && S.done[k]) return;
   cplx<double>* B = zu + (size_t)k * S.NB * S.NL;
   cplx<double>* v = B + (size_t)ib * S.NL;
   const cplx<double>* zs = S.zs + (size_t)k * S.NB;
@@ -855,8 +858,9 @@ __global__ void __launch_bounds__(256) k_gs_sub(State S, cplx<double>* __restric
 }
 
 // band ib *= SN.  Grid (nvec, NK).
-__global__ void __launch_bounds__(256) k_gs_scale(State S, cplx<double>* __restrict__ zu, int ib) {
+__global__ void __launch_bounds__(256) k_gs_scale(State S, cplx<double>* __restrict__ zu, int ib, int check_done) {
   const int k = blockIdx.y;
+  if (check_done && S.done[k]) return;
   const double f = S.sc[k * kNS + SN];
   cplx<double>* v = zu + ((size_t)k * S.NB + ib) * S.NL;
   const int p = blockIdx.x * 256 + threadIdx.x;

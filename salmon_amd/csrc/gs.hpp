@@ -186,7 +186,7 @@ static int gs_ensure(salmon_ctx* c) {
   if ((r = gs_alloc(c, s, &q.C, (size_t)s->NK * s->NB * kPanel))) return r;
   if ((r = gs_alloc(c, s, &q.W, (size_t)s->NK * s->NB * kPanel))) return r;
   if ((r = gs_alloc(c, s, &q.cnt, (size_t)s->NK * (q.ntile + 1)))) return r;
-  if ((r = gs_alloc(c, s, &q.flag, s->NK))) return r;
+  if ((r = gs_alloc(c, s, &q.fine, s->NK))) return r;
   HIPCHK(c, hipMemsetAsync(q.cnt, 0, sizeof(unsigned) * s->NK * (q.ntile + 1), c->stream));
   HIPCHK(c, hipMemsetAsync(s->cnt, 0, sizeof(unsigned) * s->NK, c->stream));
   HIPCHK(c, hipMemsetAsync(s->sc, 0, sizeof(double) * s->NK * kNS, c->stream));
@@ -345,40 +345,42 @@ static int cg_run(salmon_ctx* c, int ncg, int precond) {
 // loop's overlaps are taken against the unmodified band and the subtraction
 // is repeated once (classical Gram-Schmidt twice, equal to the reference's
 // modified form up to rounding), then the band is normalised.
-static int gram_schmidt_multi(salmon_ctx* c, cplx<double>* zu) {
+static int gram_schmidt_multi(salmon_ctx* c, cplx<double>* zu, int* skip = nullptr) {
   int r;
   if ((r = gs_ensure(c))) return r;
   GsState* s = (GsState*)c->gs;
   State S = gs_view(c, s);
+  const int check = skip ? 1 : 0;
+  if (skip) S.done = skip;
   const dim3 gv(S.nvec, s->NK), blk(256);
   for (int ib = 0; ib < s->NB; ++ib) {
     const Src v{zu + (size_t)ib * s->NL, (size_t)s->NB * s->NL, nullptr, nullptr};
     for (int pass = 0; pass < 2 && ib > 0; ++pass) {
       hipLaunchKernelGGL(k_cg_proj, dim3(s->nchunk, (ib + kJG - 1) / kJG, s->NK), blk, 0, c->stream, S,
-                         (const cplx<double>*)zu, ib, v, (int)PROJ_PLAIN, 0);
+                         (const cplx<double>*)zu, ib, v, (int)PROJ_PLAIN, check);
       LAUNCHCHK(c);
-      hipLaunchKernelGGL(k_gs_sub, gv, blk, 0, c->stream, S, zu, ib, pass == 1 ? 1 : 0);
+      hipLaunchKernelGGL(k_gs_sub, gv, blk, 0, c->stream, S, zu, ib, pass == 1 ? 1 : 0, check);
       LAUNCHCHK(c);
     }
     if (ib == 0) {
-      hipLaunchKernelGGL(k_gs_sub, gv, blk, 0, c->stream, S, zu, 0, 1);
+      hipLaunchKernelGGL(k_gs_sub, gv, blk, 0, c->stream, S, zu, 0, 1, check);
       LAUNCHCHK(c);
     }
-    hipLaunchKernelGGL(k_gs_scale, gv, blk, 0, c->stream, S, zu, ib);
+    hipLaunchKernelGGL(k_gs_scale, gv, blk, 0, c->stream, S, zu, ib, check);
     LAUNCHCHK(c);
   }
   return SALMON_OK;
 }
 
-// Gram_Schmidt_ompk in panels (gsblock.hpp); *done = 0 if a panel could not be
-// orthogonalised so (waits for the stream).
+// Gram_Schmidt_ompk in panels (gsblock.hpp); *done = 0 if a panel of some k point could
+// not be orthogonalised so, whose fine flag is then zero (waits for the stream).
 static int gram_schmidt_panels(salmon_ctx* c, cplx<double>* zu, int* done) {
   int r;
   if ((r = gs_ensure(c))) return r;
   GsState* s = (GsState*)c->gs;
   GsBlock b = s->gsb;
   b.zu = zu;
-  HIPCHK(c, hipMemsetAsync(b.flag, 0, sizeof(int) * b.NK, c->stream));
+  HIPCHK(c, hipMemsetAsync(b.fine, 1, sizeof(int) * b.NK, c->stream));
   for (int j0 = 0; j0 < b.NB; j0 += kPanel) {
     const int np = std::min(kPanel, b.NB - j0);
     for (int round = 0; round < 2; ++round) {
@@ -388,10 +390,10 @@ static int gram_schmidt_panels(salmon_ctx* c, cplx<double>* zu, int* done) {
       LAUNCHCHK(c);
     }
   }
-  std::vector<int> flag(b.NK);
-  HIPCHK(c, hipMemcpyAsync(flag.data(), b.flag, sizeof(int) * b.NK, hipMemcpyDeviceToHost, c->stream));
+  std::vector<int> fine(b.NK);
+  HIPCHK(c, hipMemcpyAsync(fine.data(), b.fine, sizeof(int) * b.NK, hipMemcpyDeviceToHost, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
-  *done = std::all_of(flag.begin(), flag.end(), [](int f) { return f == 0; });
+  *done = std::all_of(fine.begin(), fine.end(), [](int f) { return f != 0; });
   return SALMON_OK;
 }
 

@@ -15,8 +15,9 @@
 // finished bands: it also sees what no pivot of R shows by itself, bands that each
 // keep a part of their norm but lose it in turn (b_j = e_{j-1} + e_j / 30: every
 // pivot 1e-3, and twelve of them dependent to rounding).  A panel past kGsbCond, or
-// one that is not finite, sets its k point's flag before it changes: the k point's
-// bands stay as they are from there on, and the caller runs the band-by-band form.
+// one that is not finite, clears its k point's flag before it changes: the k point's
+// bands stay as they are from there on, and the caller runs the band-by-band form for
+// such k points.
 // Up to the limit the results differ from that form's by eps * kappa, 1e-12.
 //
 // Per panel round that is two launches for the finished bands' bytes read twice
@@ -43,7 +44,7 @@ struct GsBlock {
   cplx<double>* C;      // (NK, NB, 16) overlaps of the panel with bands 0 .. j0 + np - 1
   cplx<double>* W;      // (NK, NB, 16)
   unsigned* cnt;        // (NK, tiles + 1) arrivals, zero between launches
-  int* flag;            // (NK) nonzero: a panel could not be orthogonalised; the k point's bands stay from there on
+  int* fine;            // (NK) zero: a panel could not be orthogonalised; the k point's bands stay from there on
   int NK, NB, NL, nchunk, chunk, ntile;
   double Hxyz;
 };
@@ -85,7 +86,7 @@ __global__ void __launch_bounds__(256) k_gsb_overlap(GsBlock b, int j0, int np) 
   const int k = blockIdx.z, tile = blockIdx.y, c = blockIdx.x, t = threadIdx.x;
   const int lane = t & (kWave - 1), wv = t / kWave, lg = lane >> 4, li = lane & 15;
   const int nt = gridDim.y, ni = j0 + np;
-  if (b.flag[k]) return;  // (set by an earlier launch: all of the k point's blocks leave)
+  if (!b.fine[k]) return;  // (cleared by an earlier launch: all of the k point's blocks leave)
   const cplx<double>* Z = b.zu + (size_t)k * b.NB * b.NL;
   // bands past the tile's or the panel's last: its last, weighted by zero
   const int ia = tile * 16 + li, ib = j0 + li;
@@ -214,7 +215,7 @@ __global__ void __launch_bounds__(256) k_gsb_overlap(GsBlock b, int j0, int np) 
   }
   __syncthreads();
   if (!((cond[0] + cond[1]) + (cond[2] + cond[3]) <= kGsbCond)) {
-    if (t == 0) b.flag[k] = 1;
+    if (t == 0) b.fine[k] = 0;
     return;
   }
   cplx<double>* W = b.W + (size_t)k * b.NB * 16;
@@ -242,7 +243,7 @@ __global__ void __launch_bounds__(256) k_gsb_overlap(GsBlock b, int j0, int np) 
 __global__ void __launch_bounds__(256) k_gsb_apply(GsBlock b, int j0, int np) {
   const int k = blockIdx.y, t = threadIdx.x;
   const int lane = t & (kWave - 1), wv = t / kWave, lg = lane >> 4, li = lane & 15;
-  if (b.flag[k]) return;
+  if (!b.fine[k]) return;
   const int p = blockIdx.x * 64 + wv * 16 + li, pc = min(p, b.NL - 1), n = j0 + np;
   cplx<double>* Z = b.zu + (size_t)k * b.NB * b.NL;
   const cplx<double>* W = b.W + (size_t)k * b.NB * 16;

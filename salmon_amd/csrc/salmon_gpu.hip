@@ -489,10 +489,11 @@ int gram_schmidt_multi_fwd(salmon_ctx* c, cplx<double>* zu) {
   // and 4 bands of 16^3 at 8 k points take 82, 84, 85 and 85 us in panels, 12, 40, 66
   // and 92 band by band (8x21x32 at 15 k points 82, 86, 89, 89 and 27, 48, 80, 111)
   if (c->NB > 3 && ((r = gram_schmidt_panels(c, zu, &done)) || done)) return r;
-  // few, nearly dependent (or not finite) bands: band by band
+  // few bands, and the k points of nearly dependent (or not finite) ones: band by band
   GsState* s = (GsState*)c->gs;
+  int* skip = c->NB > 3 ? s->gsb.fine : nullptr;
   const long key[4] = {(long)(uintptr_t)zu, c->NB, c->NK, 0};
-  return graph_run(c, s->g_gs, key, [&]() { return gram_schmidt_multi(c, zu); });
+  return graph_run(c, s->g_gs, key, [&]() { return gram_schmidt_multi(c, zu, skip); });
 }
 }  // namespace
 

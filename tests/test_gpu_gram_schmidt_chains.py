@@ -80,3 +80,22 @@ def test_mild_chains(step, n):
     z = run(s)
     assert overlap_error(s, z) < 1e-13
     assert rel(z, synth.gram_schmidt(s.zu, s.Hxyz)) < 1e-11
+
+
+def test_other_k_points_are_left_alone():
+    """A k point left to the band-by-band form changes nothing of the others: eager, captured and replayed calls."""
+    s = system(9, seed=9)
+    good = run(s)
+    s.zu[1, 6] = s.zu[1, 2] * (0.3 + 0.9j) + 1e-6 * s.zu[1, 6]
+    with gpu.Context(s, gpu.FP64) as c:
+        for call in range(3):
+            c.put_orbitals(s.zu)
+            c.gram_schmidt()
+            z = c.get_orbitals()
+            assert np.array_equal(z[0], good[0]), call
+            assert overlap_error(s, z) < 1e-13
+        s.zu[0], s.zu[1] = s.zu[1].copy(), s.zu[0].copy()  # the replayed launches follow the flags
+        c.put_orbitals(s.zu)
+        c.gram_schmidt()
+        z1 = c.get_orbitals()
+        assert np.array_equal(z1[1], good[0]) and np.array_equal(z1[0], z[1])
