@@ -153,7 +153,8 @@ static size_t sweep_lds_bytes(const Sys<T>& y, const std::array<int, 2>& sh) {
 // its x points per thread and atoms per wave, the sweep by planes, column length,
 // team size and passes over the sphere points, and by how full the chip is.  The
 // lines, 1.1 and in complex64 1.25, are where runs of ten steps (which the resident
-// kernel needs fewer launches for) took as long either way.  Without the comparison 14^3 x 1024 orbitals took 194 us a hamiltonian call
+// kernel needs fewer launches for) took as long either way; with several shapes, a
+// launch after another, 0.9.  Without the comparison 14^3 x 1024 orbitals took 194 us a hamiltonian call
 // in FP64 where the sweep takes 144, 31x8x9 x 1024 193 and 138; 12^3 x 1024 104
 // and 119.
 template <typename T>
@@ -197,7 +198,7 @@ static bool resident_pays(const salmon_batch* b, const std::vector<Sys<T>>& S, i
     mean += (chain * (f64 ? 1.45 : 1.64) + kb) * ((S[i].NKB + teams - 1) / teams) / items;
     most = std::max(most, chain * (1.0 + (f64 ? 0.45 : 0.64) * rest / slots) + kb);
   }
-  return res <= (f64 ? 1.1 : 1.25) * (full * mean + (rest ? most : 0.0));
+  return res <= (cls.size() > 1 ? 0.9 : f64 ? 1.1 : 1.25) * (full * mean + (rest ? most : 0.0));
 }
 
 template <typename T>

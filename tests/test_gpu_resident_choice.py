@@ -37,3 +37,25 @@ def test_choice(N, nk, nb, natoms, prec, resident):
             out.append(r)
     for x in out[0]:
         assert rel(out[0][x], out[1][x]) < TOL[prec], x
+
+
+@pytest.mark.parametrize("prec", [gpu.FP64, gpu.MIXED])
+@pytest.mark.parametrize("grids,resident", [
+    ([(8, 8, 8), (8, 9, 10), (9, 10, 11), (10, 10, 10), (11, 11, 11), (12, 12, 12), (12, 10, 8), (13, 13, 13), (14, 14, 14),
+      (15, 15, 15), (8, 16, 16), (16, 8, 16), (16, 12, 12), (24, 8, 8), (31, 8, 9), (10, 12, 14)], 0),
+    ([(8, 8, 8), (12, 12, 12), (16, 16, 16)], 1)])
+def test_choice_for_batches_of_shapes(grids, resident, prec):
+    """Many shapes would be as many launches of the resident kernel, one after another; few are not too many."""
+    systems = [cell(N, nk=2, nb=2, natoms=2, seed=i) for i, N in enumerate(grids)]
+    ac = synth.acos2_pulse(3, 0.08, 0.05, 0.3, 4.0)
+    ctx = [gpu.Context(s, prec) for s in systems]
+    with gpu.Batch(ctx, prec) as b:
+        r = b.rt_run(ac, 2, 0.08)
+        assert b.resident() == resident
+    for i, s in enumerate(systems):
+        ctx[i].close()
+        with gpu.Context(s, prec) as c:
+            c.set_path(gpu.PATH_STREAMED)
+            q = c.rt_run(ac, 2, dt=0.08)
+        for x in ("J", "E", "norm"):
+            assert rel(r[x][i], q[x]) < TOL[prec], (i, x)
