@@ -82,7 +82,14 @@ __device__ __forceinline__ void plane(int NA, int NB, int nl, const double* twa,
     // long lines leave few sums a tile: neighbouring lanes share each (ten planes of
     // 200x200 1.47 -> 1.05 ms)
     int parts = 1;
-    while (parts < 8 && 2 * parts * nb * na <= 256) parts *= 2;
+    while (parts < 8 && 2 * parts * nb * na <= 256 && NA > 32 * parts) parts *= 2;
+    if (parts == 1) {
+      for (int i = t; i < nb * na; i += 256) {
+        const int b = i / na, a = i - b * na;
+        mid[(b0 + b) * na + a] = line_sum(tile + b * NA, 1, NA, a0 + a, wa, sgn);
+      }
+      continue;
+    }
     for (int i = t; i < nb * na * parts; i += 256) {
       const int o = i / parts, b = o / na, a = o - b * na;
       cplx<double> v = line_sum(tile + b * NA, 1, NA, a0 + a, wa, sgn, i - o * parts, parts);
