@@ -208,7 +208,8 @@ int salmon_gpu_set_pcnet(salmon_ctx *ctx, salmon_pcnet *net);
  * (from the third on) that lowers the band-energy sum by less than
  * stall_ratio times the previous sweep's drop. */
 int salmon_gpu_set_pc_handover(salmon_ctx *ctx, int max_learned_sweeps, double stall_ratio);
-/* No counterpart in the reference.  CG and Gram-Schmidt calls run through a
+/* No counterpart in the reference.  CG calls and Gram-Schmidt in its band-by-band
+ * form (up to 3 bands, or nearly dependent ones) run through a
  * graph cache (captured on the second call with the same arguments, replayed
  * after); enable = 0 runs them eagerly.  While a context's stream is being
  * captured, a HIP call of another host thread that touches the legacy stream
@@ -258,8 +259,8 @@ int salmon_gpu_rt_run(salmon_ctx *ctx, const double *ac, int nsteps, double dt, 
  * default) takes the sweep when every system fits it, and in its place the
  * resident kernel -- every orbital in the LDS of one workgroup, up to 32 steps
  * per launch -- when every system fits that too (orbital and sphere points
- * within 160 KB, up to four projectors per atom) and the batch has at most
- * four orbitals per compute unit.  salmon_gpu_batch_kernel reports the kind in
+ * within 160 KB, up to four projectors per atom), the batch has at most
+ * four orbitals per compute unit and the sweep is not expected to be faster.  salmon_gpu_batch_kernel reports the kind in
  * use after tune (-1 before; SALMON_BATCH_SWEEP also for the resident kernel),
  * salmon_gpu_batch_resident whether it is the resident kernel (1, 0; -1 before
  * tune).  SALMON_BATCH_SWEEP asked for is the sweep itself.  For the phase kernel

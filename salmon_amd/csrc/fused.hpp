@@ -1222,7 +1222,7 @@ static int fused_step(salmon_ctx* c, const double* amid, const double* aobs, dou
   const int per_cu = std::min(sizeof(T) == 8 ? 1 : 2, by_regs);
   // orbitals per workgroup (of one k point): the least rounds * (orbitals + set-up)
   // over the rounds of resident workgroups.  A complex64 orbital takes 20 us and the
-  // set-up (phases, tables into LDS) 19, FP64 45 and about as much: 64 k x 32
+  // set-up (phases, tables into LDS) 19, FP64 45 and about 20: 64 k x 32
   // complex64 orbitals in one round of 8 each instead of two of 4, 201 -> 188 us.
   int bpw = 1;
   long best = -1;
