@@ -142,10 +142,11 @@ struct Src {
 //   PROJ_GRAM   stores row ib of G from the stored band ib, and row ib of
 //               both inverses: M(ib, l) = -sum_{l<=q<ib} G(ib, q) M(q, l)
 //               (unit diagonal implicit).
-//   PROJ_PLAIN  b itself (Gram-Schmidt), for any number of bands.
+//   PROJ_PLAIN  b itself (Gram-Schmidt).
+// ib is at most kCgMaxNB (PROJ_PLAIN takes more lower bands in several launches).
 // Grid: (nchunk, ceil(ib/kJG), NK).
 enum : int { PROJ_START = 0, PROJ_VEC = 1, PROJ_GRAM = 2, PROJ_PLAIN = 3 };
-constexpr int kCgMaxNB = 1024;  // bands of the CG, whose modes hold b in LDS
+constexpr int kCgMaxNB = 1024;
 
 __global__ void __launch_bounds__(256) k_cg_proj(State S, const cplx<double>* __restrict__ zu, int ib, Src src,
                                                  int mode, int check_done) {
@@ -257,13 +258,14 @@ __global__ void __launch_bounds__(256) k_cg_proj(State S, const cplx<double>* __
     __syncthreads();
     if (sh == 0 && v < 2 * ib) {
       for (int r = 1; r < ns; ++r) s += smem[r * nv + t];
-      // PROJ_PLAIN: coefficients against the unmodified vector, and any number of bands
-      if (mode == PROJ_PLAIN) ((double*)(S.zs + (size_t)k * S.NB))[v] = s * S.Hxyz;
-      else zv[v] = s * S.Hxyz;
+      zv[v] = s * S.Hxyz;
     }
   }
-  if (mode == PROJ_PLAIN) return;
   __syncthreads();
+  if (mode == PROJ_PLAIN) {  // coefficients against the unmodified vector
+    for (int j = t; j < ib; j += 256) S.zs[(size_t)k * S.NB + j] = zsh[j];
+    return;
+  }
   auto quad = [](double v) {
     v += dpp_mov<dpp::kQuad1032, 0xf>(v);
     return v + dpp_mov<dpp::kQuad2301, 0xf>(v);

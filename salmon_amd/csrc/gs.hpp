@@ -356,9 +356,14 @@ static int gram_schmidt_multi(salmon_ctx* c, cplx<double>* zu, int* skip = nullp
   for (int ib = 0; ib < s->NB; ++ib) {
     const Src v{zu + (size_t)ib * s->NL, (size_t)s->NB * s->NL, nullptr, nullptr};
     for (int pass = 0; pass < 2 && ib > 0; ++pass) {
-      hipLaunchKernelGGL(k_cg_proj, dim3(s->nchunk, (ib + kJG - 1) / kJG, s->NK), blk, 0, c->stream, S,
-                         (const cplx<double>*)zu, ib, v, (int)PROJ_PLAIN, check);
-      LAUNCHCHK(c);
+      for (int b0 = 0; b0 < ib; b0 += kCgMaxNB) {
+        const int nb = std::min(kCgMaxNB, ib - b0);
+        State P = S;
+        P.zs += b0;
+        hipLaunchKernelGGL(k_cg_proj, dim3(s->nchunk, (nb + kJG - 1) / kJG, s->NK), blk, 0, c->stream, P,
+                           (const cplx<double>*)zu + (size_t)b0 * s->NL, nb, v, (int)PROJ_PLAIN, check);
+        LAUNCHCHK(c);
+      }
       hipLaunchKernelGGL(k_gs_sub, gv, blk, 0, c->stream, S, zu, ib, pass == 1 ? 1 : 0, check);
       LAUNCHCHK(c);
     }
